@@ -184,7 +184,12 @@ typedef struct KarpoAttnBwdArgs {
   int64_t d_v_stride_tok, d_v_stride_head;
 } KarpoAttnBwdArgs;
 
+/* The least workspace the call runs in, and the workspace its fastest path takes (never less; the same for most
+ * calls). At head size 512 a call of one sequence without a left window bound or spans holds P and dS of a chunk of
+ * query rows (at most 4 GiB) and, over several chunks, dK and dV in fp32; karpo_attn_bwd takes that path when
+ * workspace_bytes allows it, and the path of the least workspace otherwise. */
 int karpo_attn_bwd_workspace_bytes(const KarpoAttnBwdArgs* args, size_t* bytes);
+int karpo_attn_bwd_workspace_best_bytes(const KarpoAttnBwdArgs* args, size_t* bytes);
 int karpo_attn_bwd(const KarpoAttnBwdArgs* args, void* stream);
 
 /* Bytes of device workspace karpo_attn_fwd needs for these arguments (reads only sizes and whether k_rows is set:

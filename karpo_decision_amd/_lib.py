@@ -110,6 +110,8 @@ def load() -> ctypes.CDLL:
         lib.karpo_attn_norm_rope.restype = ctypes.c_int
         lib.karpo_attn_bwd_workspace_bytes.argtypes = [P(KarpoAttnBwdArgs), P(ctypes.c_size_t)]
         lib.karpo_attn_bwd_workspace_bytes.restype = ctypes.c_int
+        lib.karpo_attn_bwd_workspace_best_bytes.argtypes = [P(KarpoAttnBwdArgs), P(ctypes.c_size_t)]
+        lib.karpo_attn_bwd_workspace_best_bytes.restype = ctypes.c_int
         lib.karpo_attn_bwd.argtypes = [P(KarpoAttnBwdArgs), ctypes.c_void_p]
         lib.karpo_attn_bwd.restype = ctypes.c_int
         lib.karpo_attn_device_status.argtypes = [P(KarpoAttnArgs), ctypes.c_void_p, P(ctypes.c_int32)]

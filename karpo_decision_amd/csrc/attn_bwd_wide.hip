@@ -1,0 +1,444 @@
+// The backward at head size 512 for one sequence (a training sequence's global layer) as two matrix-product kernels
+// per chunk of query rows, with P and dS of the chunk held in the workspace as bf16 (the precision at which they enter
+// the matrix products in every backward kernel here):
+//   1. bwd_wide_ds_kernel: S = Q K^T and dP = dO V^T of a tile of 256 rows x 128 keys, then P and dS, stored;
+//   2. bwd_wide_grad_kernel: dQ = dS K, dK = dS^T Q and dV = P^T dO, 256 x 256 outputs per workgroup.
+// Why: at this head size a wave cannot hold the operands and accumulators of a fused tile (attn_bwd_pair.hip: pairs
+// of waves that exchange partial sums through LDS, one wave per SIMD, three barriers per 32-row step, 24-26% of the
+// MFMA rate), and it computes S and dP twice (seven products). P and dS cost 10 bytes of traffic per visible pair and
+// 5,120 FLOPs need them, so keeping them takes less time than either the recomputation or the exchange: five products,
+// each a plain tiled matrix product with every accumulator in one wave's registers. Measured against the wave pairs
+// (32 / 4 heads, causal, MI355X): 497 -> 140 us at 512 rows, 2.09 -> 0.83 ms at 2,048, 12.4 -> 8.0 ms at 8,192, 48.1 ->
+// 29.9 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
+// call takes this path when the workspace has room for a chunk of 256 rows.
+//
+// P and dS in the workspace: per head [key block of 16][chunk of 8 rows][16 keys][8 rows] bf16, the 16 keys of a
+// 256-byte run XOR-swizzled by the chunk index as in the S layout (mfma_common.h): the layout in which a tile is read
+// from LDS, so a copy instruction moves 1 KiB of consecutive bytes. A lane of kernel 1 holds one key's scores of 8
+// consecutive rows (the MFMA's A rows are taken in key_row order) and stores them as one 16-byte chunk; dK and dV read
+// those chunks directly as MFMA operands, dQ reads the same tile transposed.
+//
+// Chunks of rows run in ascending order. dQ of a chunk's rows is complete within it; dK and dV go on from one chunk to
+// the next in fp32 (workspace, in the accumulators' register order) and are rounded once, in the last chunk.
+// Every sum has a fixed order (no atomics): repeated calls are bitwise equal.
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stdint.h>
+
+#include "bwd_common.h"
+#include "internal.h"
+#include "karpo_attn.h"
+#include "mfma_common.h"
+#include "plan_common.h"
+
+namespace karpo {
+
+constexpr int kWideD = 512;
+constexpr int kWideThreads = 512;               // eight waves
+constexpr int kDsRows = 256, kDsKeys = 128;     // kernel 1's tile
+constexpr int kDsStep = 64;                     // elements of D per step
+constexpr int kGradTile = 256, kGradStep = 64;  // kernel 2's outputs (both ways) and contraction step
+
+// The sequence's bounds, clamped to the call's rows.
+struct WideSeq {
+  int qa, lq, ka, lk;
+  __device__ __forceinline__ explicit WideSeq(const BwdWideParams& w) {
+    qa = w.b.q_cu[0];
+    ka = w.b.k_cu[0];
+    lq = min(w.b.q_cu[1], (int)w.b.total_q) - qa;
+    lk = min(w.b.k_cu[1], w.total_k) - ka;
+  }
+  // The first query row that sees `key` (no left bound): key - right <= row + lk - lq.
+  __device__ __forceinline__ int first_row(int right, int key) const {
+    if (right < 0) return 0;
+    const int64_t r = (int64_t)key - right - (lk - lq);
+    return r < 0 ? 0 : (int)min(r, (int64_t)INT32_MAX);
+  }
+};
+
+// Work index -> head with XCD w % 8 given heads that are neighbours (the same key/value head) where the count allows.
+__device__ __forceinline__ int spread_head(int i, int n) { return n % 8 == 0 ? (i % 8) * (n / 8) + i / 8 : i; }
+
+// s_barrier after the wave's own LDS accesses, without the fence of __syncthreads (which waits for every copy in
+// flight): the copies a step needs are waited for by count.
+__device__ __forceinline__ void step_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// ---- kernel 1: P and dS of 256 rows x 128 keys of one head (eight waves of 64 x 64)
+__global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_ds_kernel(BwdWideParams w) {
+  constexpr int STEPS = kWideD / kDsStep;  // per product
+  constexpr int AT = kDsRows * kDsStep * 2, BT = kDsKeys * kDsStep * 2;
+  __shared__ __attribute__((aligned(1024))) char a0_s[AT], a1_s[AT], a2_s[AT];
+  __shared__ __attribute__((aligned(1024))) char b0_s[BT], b1_s[BT], b2_s[BT];
+  __shared__ __attribute__((aligned(16))) float st_s[2][kDsRows];  // the rows' log2 LSE and -D
+
+  const BwdParams& p = w.b;
+  const WideSeq s(w);
+  const int key_tiles = w.keys / kDsKeys;
+  const int head = spread_head(blockIdx.x % p.heads, p.heads);
+  const int rest = blockIdx.x / p.heads;
+  const int rt = rest / key_tiles, kt = rest - rt * key_tiles;
+  const int r0 = w.r_begin + rt * kDsRows, k0 = kt * kDsKeys;
+  const int k_pair = k0 & ~(kGradTile - 1);  // kernel 2 reads keys in tiles of 256
+  if (r0 >= s.lq || k_pair >= s.lk || r0 + kDsRows <= s.first_row(p.right, k_pair)) return;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const int wr = wave >> 1, wc = wave & 1;
+  // this lane's chunk (rows rt*256 + wr*64 + rb*32 + kc*16 + half*8 .. +8) of key k0 + wc*64 + cb*32 + col
+  char* const out_p = (char*)(w.p + (int64_t)head * w.keys * w.rows);
+  char* const out_s = (char*)(w.ds + (int64_t)head * w.keys * w.rows);
+  const uint32_t run = (uint32_t)(w.rows / 8) * 256u;  // bytes per block of 16 keys
+  const uint32_t out_base =
+      (uint32_t)(kt * 8 + wc * 4 + (col >> 4)) * run + (uint32_t)(rt * 32 + wr * 8 + half) * 256u;
+  const uint32_t out_key[2] = {(uint32_t)((col & 15) ^ (half << 2)) * 16u,
+                               (uint32_t)((col & 15) ^ ((2 + half) << 2)) * 16u};
+  if (k0 >= s.lk || r0 + kDsRows <= s.first_row(p.right, k0)) {  // nothing seen, but read by kernel 2
+    const u32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int kc = 0; kc < 2; ++kc) {
+          const uint32_t at = out_base + (uint32_t)cb * 2u * run + (uint32_t)(rb * 4 + kc * 2) * 256u + out_key[kc];
+          *(u32x4*)(out_p + at) = zero;
+          *(u32x4*)(out_s + at) = zero;
+        }
+    return;
+  }
+
+  {
+    const int row = r0 + (tid & 255), which = tid >> 8;
+    st_s[which][tid & 255] = row < s.lq ? p.stats[((int64_t)head * 2 + which) * p.total_q + s.qa + row]
+                                        : (which ? 0.f : INFINITY);  // a row past the sequence has P = 0
+  }
+  const int kvh = head / p.group;
+  const uint16_t* const q = p.q + (int64_t)(s.qa + r0) * p.sq_t + (int64_t)head * p.sq_h;
+  const uint16_t* const o = p.dout + (int64_t)(s.qa + r0) * p.sdo_t + (int64_t)head * p.sdo_h;
+  const uint16_t* const k = p.k + (int64_t)(s.ka + k0) * p.sk_t + (int64_t)kvh * p.sk_h;
+  const uint16_t* const v = p.v + (int64_t)(s.ka + k0) * p.sv_t + (int64_t)kvh * p.sv_h;
+  const int rows = min(s.lq - r0, kDsRows), keys = min(s.lk - k0, kDsKeys);
+  // tiles in the K layout of 64 columns: wave w copies A rows 32w .. +32 (four 1 KiB blocks: 16 rows x 64 B) and B
+  // rows 16w .. +16 (two)
+  const int lrow = lane & 15;
+  const uint32_t lcol = (uint32_t)(lane >> 4) * 16u;
+  const uint32_t q_off = (uint32_t)((wave * 32 + lrow) * (int)p.sq_t) * 2u + lcol;
+  const uint32_t o_off = (uint32_t)((wave * 32 + lrow) * (int)p.sdo_t) * 2u + lcol;
+  const uint32_t k_off = (uint32_t)((wave * 16 + lrow) * (int)p.sk_t) * 2u + lcol;
+  const uint32_t v_off = (uint32_t)((wave * 16 + lrow) * (int)p.sv_t) * 2u + lcol;
+  auto copy = [&](int step, KA_LDS char* a, KA_LDS char* b) {
+    const bool second = step >= STEPS;
+    const int at = (second ? step - STEPS : step) * kDsStep;
+    const uint16_t* const as = (second ? o : q) + at;
+    const uint16_t* const bs = (second ? v : k) + at;
+    const int a_t = (int)(second ? p.sdo_t : p.sq_t) * 2, b_t = (int)(second ? p.sv_t : p.sk_t) * 2;
+    const uint32_t a_off = second ? o_off : q_off, b_off = second ? v_off : k_off;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      dma_16b(as, rows * a_t, a + (wave * 4 + r) * 1024, a_off + (uint32_t)((r >> 1) * 16 * a_t) + (r & 1) * 64u);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) dma_16b(bs, keys * b_t, b + (wave * 2 + r) * 1024, b_off + r * 64u);
+  };
+  const int arow = key_row(col);
+  const int a_read = ((wr * 4 + (arow >> 4)) * 8 + half) * 256 + (arow & 15) * 16;  // + rb * 4096 + kk * 512
+  const int b_read = ((wc * 4 + (col >> 4)) * 8 + half) * 256 + (col & 15) * 16;    // + cb * 4096 + kk * 512
+
+  f32x16 st[2][2], dp[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      st[i][j] = f32x16{};
+      dp[i][j] = f32x16{};
+    }
+  auto products = [&](f32x16 (&acc)[2][2], const KA_LDS char* a, const KA_LDS char* b) {
+#pragma unroll
+    for (int kk = 0; kk < kDsStep / 16; ++kk) {
+      bf16x8 x[2], y[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        x[i] = *(const KA_LDS bf16x8*)(a + a_read + i * 4096 + kk * 512);
+        y[i] = *(const KA_LDS bf16x8*)(b + b_read + i * 4096 + kk * 512);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  KA_LDS char* const at[3] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s, (KA_LDS char*)a2_s};
+  KA_LDS char* const bt[3] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s, (KA_LDS char*)b2_s};
+  // a ring of three buffers: two steps of copies in flight
+  copy(0, at[0], bt[0]);
+  copy(1, at[1], bt[1]);
+  wait_vmcnt<6>();
+  step_barrier();
+#pragma unroll
+  for (int i = 0; i < 2 * STEPS; ++i) {
+    if (i + 2 < 2 * STEPS) copy(i + 2, at[(i + 2) % 3], bt[(i + 2) % 3]);
+    __builtin_amdgcn_sched_barrier(0);  // the copies are issued first
+    products(i < STEPS ? st : dp, at[i % 3], bt[i % 3]);
+    if (i + 1 < 2 * STEPS) {
+      if (i + 2 < 2 * STEPS) wait_vmcnt<6>(); else wait_vmcnt<0>();
+      step_barrier();
+    }
+  }
+
+  const float c = p.c;
+  const bool whole = k0 + kDsKeys <= s.lk && r0 >= s.first_row(p.right, k0 + kDsKeys - 1);
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+      const int lr = wr * 64 + rb * 32 + kc * 16 + half * 8;  // the chunk's first row in the tile
+      const f32x4 l0 = *(const f32x4*)&st_s[0][lr], l1 = *(const f32x4*)&st_s[0][lr + 4];
+      const f32x4 d0 = *(const f32x4*)&st_s[1][lr], d1 = *(const f32x4*)&st_s[1][lr + 4];
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        float x[8], y[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+          x[t] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[rb][cb][kc * 8 + t], c, -(t < 4 ? l0[t] : l1[t - 4])));
+          y[t] = x[t] * (dp[rb][cb][kc * 8 + t] + (t < 4 ? d0[t] : d1[t - 4]));
+        }
+        if (!whole) {
+          const int key = k0 + wc * 64 + cb * 32 + col;
+          const int first = key < s.lk ? s.first_row(p.right, key) : INT32_MAX;
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            const bool vis = r0 + lr + t >= first;
+            x[t] = vis ? x[t] : 0.f;
+            y[t] = vis ? y[t] : 0.f;
+          }
+        }
+        const uint32_t to = out_base + (uint32_t)cb * 2u * run + (uint32_t)(rb * 4 + kc * 2) * 256u + out_key[kc];
+        u32x4 px, dx;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          px[t] = pack_bf16(x[2 * t], x[2 * t + 1]);
+          dx[t] = pack_bf16(y[2 * t], y[2 * t + 1]);
+        }
+        *(u32x4*)(out_p + to) = px;
+        *(u32x4*)(out_s + to) = dx;
+      }
+    }
+}
+
+// ---- kernel 2: a 256 x 256 output (256 columns of D, and 256 query rows of dQ or 256 keys of dK or dV) per
+// workgroup, eight waves of 128 (D) x 64
+template <bool DQ>
+__device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq& s, int item, KA_LDS char* const (&at)[2],
+                                          KA_LDS char* const (&bt)[2]) {
+  const BwdParams& p = w.b;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 31, half = lane >> 5;
+  const int wd = wave >> 2, wn = wave & 3;
+  const uint32_t run = (uint32_t)(w.rows / 8) * 256u;
+  const int r_end = min(s.lq, w.r_begin + w.rows);
+
+  int head, dhalf, n0, which = 0, steps, first = 0;  // n0: the first query row (dQ, from the chunk's first) or key
+  bool carry = false, last = true;
+  if constexpr (DQ) {
+    head = spread_head(item % p.heads, p.heads);
+    const int rest = item / p.heads;
+    dhalf = rest & 1;
+    n0 = (w.rows / kGradTile - 1 - (rest >> 1)) * kGradTile;  // the rows that see most keys first
+    const int row = w.r_begin + n0;
+    if (row >= s.lq) return;
+    const int top = min(row + kGradTile, s.lq) - 1;
+    const int64_t seen = p.right < 0 ? s.lk : (int64_t)top + (s.lk - s.lq) + p.right + 1;
+    const int khi = (int)max((int64_t)0, min(seen, (int64_t)s.lk));
+    steps = (khi + kGradStep - 1) / kGradStep;
+  } else {
+    const int kinds = 2 * (p.heads / p.group);
+    const int kind = item % kinds, rest = item / kinds;
+    head = kind >> 1;  // the key/value head
+    which = kind & 1;  // 0: dK, 1: dV
+    dhalf = rest & 1;
+    n0 = (rest >> 1) * kGradTile;
+    if (n0 >= s.lk) return;
+    last = s.lq <= w.r_begin + w.rows && (s.lq > w.r_begin || w.r_begin == 0);
+    const int seen = s.first_row(p.right, n0);
+    first = max(seen, w.r_begin) & ~(kGradStep - 1);
+    carry = seen < w.r_begin;
+    steps = first < r_end ? (r_end - first + kGradStep - 1) / kGradStep : 0;
+    if (steps == 0 && !(last && !carry)) return;  // no row of the chunk sees these keys
+  }
+
+  // copies: the A tile (64 keys or query rows x 256 columns of D, S layout): wave w copies columns (w & 1) * 128 ..
+  // of rows (w >> 1) * 16 .. +16; the B tile: dQ 64 keys x 256 rows, dK / dV 256 keys x 64 rows of P or dS
+  const int64_t a_t = DQ ? p.sk_t : which ? p.sdo_t : p.sq_t;
+  const int64_t a_h = which ? p.sdo_h : p.sq_h;
+  const uint32_t a_off = (uint32_t)(((wave >> 1) * 16 + ((lane & 15) ^ ((lane >> 4) << 2))) * (int)a_t) * 2u +
+                         (uint32_t)(wave & 1) * 256u + (uint32_t)(lane >> 4) * 16u;
+  const int64_t head_bytes = (int64_t)w.keys * w.rows * 2;
+  const uint16_t* a_src;
+  const char* b_src;
+  int left_rows, in_head = 0;
+  uint32_t b_off[2];
+  if constexpr (DQ) {
+    a_src = p.k + (int64_t)s.ka * a_t + (int64_t)(head / p.group) * p.sk_h + dhalf * 256;
+    left_rows = s.lk;
+    b_src = (const char*)w.ds + head * head_bytes + (int64_t)(n0 / 8) * 256;
+    b_off[0] = (uint32_t)(wave >> 1) * run + (uint32_t)(wave & 1) * 4096u + (uint32_t)lane * 16u;
+    b_off[1] = b_off[0] + 2048u;
+  } else {
+    a_src = (which ? p.dout : p.q) + (int64_t)(s.qa + first) * a_t + (int64_t)head * p.group * a_h + dhalf * 256;
+    left_rows = s.lq - first;
+    b_src = (const char*)(which ? w.p : w.ds) + (int64_t)head * p.group * head_bytes + (int64_t)(n0 / 16) * run +
+            (int64_t)((first - w.r_begin) / 8) * 256;
+    b_off[0] = (uint32_t)(wave * 2) * run + (uint32_t)lane * 16u;
+    b_off[1] = b_off[0] + run;
+  }
+  const int64_t a_step = (int64_t)kGradStep * a_t;
+  const int64_t b_step = DQ ? (int64_t)(kGradStep / 16) * run : (int64_t)(kGradStep / 8) * 256;
+  const int b_bytes = (int)((DQ ? kGradStep / 16 : kGradTile / 16) * run);
+  const int64_t a_wrap = a_h - steps * a_step, b_wrap = head_bytes - steps * b_step;
+  const int top_rows = left_rows;
+  auto copy = [&](KA_LDS char* a, KA_LDS char* b) {
+    const int bytes = min(left_rows, kGradStep) * (int)a_t * 2;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      dma_16b(a_src, bytes, a + (wave * 4 + r) * 1024, a_off + r * 64u);
+      dma_16b((const uint16_t*)b_src, b_bytes, b + (wave * 4 + r) * 1024, b_off[r >> 1] + (r & 1) * 1024u);
+    }
+    a_src += a_step;
+    b_src += b_step;
+    left_rows -= kGradStep;
+    if constexpr (!DQ) {
+      if (++in_head == steps) {  // the group's next head
+        in_head = 0;
+        a_src += a_wrap;
+        b_src += b_wrap;
+        left_rows = top_rows;
+      }
+    }
+  };
+  const int t_read[2] = {s_tr_base(lane, 0), s_tr_base(lane, 1)};  // + kc * 8192 + 32-column block * 1024
+  // dK / dV: chunk kc*2 + half of key wn*64 + j*32 + col
+  const int x_read[2] = {((wn * 4 + (col >> 4)) * 8 + half) * 256 + ((col & 15) ^ (half << 2)) * 16,
+                         ((wn * 4 + (col >> 4)) * 8 + 2 + half) * 256 + ((col & 15) ^ ((2 + half) << 2)) * 16};
+
+  f32x16 acc[4][2];
+  f32x4* const kept = (f32x4*)w.acc + (int64_t)item * 32 * kWideThreads + tid;
+  const bool any = !DQ && carry;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      acc[i][j] = f32x16{};
+      if (any) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 x = kept[((i * 2 + j) * 4 + g) * kWideThreads];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][g * 4 + e] = x[e];
+        }
+      }
+    }
+
+  auto tr = [&](const KA_LDS char* t, int at) {
+    bf16x4 x[2];
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr)
+      x[rr] = __builtin_bit_cast(bf16x4,
+                                 __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(t + t_read[rr] + at)));
+    return __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  const int total = DQ ? steps : steps * p.group;
+  auto step = [&](int n, const KA_LDS char* a, const KA_LDS char* b, KA_LDS char* an, KA_LDS char* bn) {
+    if (n + 1 < total) copy(an, bn);
+    __builtin_amdgcn_sched_barrier(0);  // the copies are issued first
+#pragma unroll
+    for (int kc = 0; kc < kGradStep / 16; ++kc) {
+      bf16x8 x[4], y[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if constexpr (DQ) y[j] = tr(b, kc * 8192 + wn * 2048 + j * 1024);
+        else y[j] = *(const KA_LDS bf16x8*)(b + x_read[kc & 1] + (kc >> 1) * 1024 + j * 4096);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = tr(a, kc * 8192 + wd * 4096 + i * 1024);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
+    }
+    wait_vmcnt<0>();
+    step_barrier();
+  };
+  if (total > 0) copy(at[0], bt[0]);
+  wait_vmcnt<0>();
+  __syncthreads();
+  int n = 0;
+  for (; n + 1 < total; n += 2) {
+    step(n, at[0], bt[0], at[1], bt[1]);
+    step(n + 1, at[1], bt[1], at[0], bt[0]);
+  }
+  if (n < total) step(n, at[0], bt[0], at[1], bt[1]);
+
+  if (!DQ && !last) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          kept[((i * 2 + j) * 4 + g) * kWideThreads] =
+              f32x4{acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
+    return;
+  }
+  // lane (col, half) holds d = dhalf*256 + wd*128 + i*32 + (reg/4)*8 + half*4 + reg%4 of row / key wn*64 + j*32 + col
+  const float scale = DQ || which == 0 ? p.scale : 1.f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int at_n = n0 + wn * 64 + j * 32 + col;
+    const bool valid = DQ ? w.r_begin + at_n < s.lq : at_n < s.lk;
+    uint16_t* to;
+    if constexpr (DQ) to = p.dq + (int64_t)(s.qa + w.r_begin + at_n) * p.sdq_t + (int64_t)head * p.sdq_h;
+    else to = which ? p.dv + (int64_t)(s.ka + at_n) * p.sdv_t + (int64_t)head * p.sdv_h
+                    : p.dk + (int64_t)(s.ka + at_n) * p.sdk_t + (int64_t)head * p.sdk_h;
+    to += dhalf * 256 + wd * 128 + half * 4;
+    if (!valid) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        u32x2 x;
+        x[0] = pack_bf16(acc[i][j][g * 4] * scale, acc[i][j][g * 4 + 1] * scale);
+        x[1] = pack_bf16(acc[i][j][g * 4 + 2] * scale, acc[i][j][g * 4 + 3] * scale);
+        *(u32x2*)(to + i * 32 + g * 8) = x;
+      }
+  }
+}
+
+__global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_grad_kernel(BwdWideParams w) {
+  constexpr int TILE = kGradStep * kGradTile * 2;
+  __shared__ __attribute__((aligned(1024))) char a0_s[TILE], a1_s[TILE], b0_s[TILE], b1_s[TILE];
+  KA_LDS char* const at[2] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s};
+  KA_LDS char* const bt[2] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s};
+  const WideSeq s(w);
+  const int dq_items = w.rows / kGradTile * 2 * w.b.heads;
+  if ((int)blockIdx.x < dq_items) wide_grad<true>(w, s, blockIdx.x, at, bt);
+  else wide_grad<false>(w, s, blockIdx.x - dq_items, at, bt);
+}
+
+hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream) {
+  const int kv_heads = w.b.heads / w.b.group;
+  const int64_t ds_items = (int64_t)(w.rows / kDsRows) * (w.keys / kDsKeys) * w.b.heads;
+  const int64_t grad_items = (int64_t)(w.rows / kGradTile) * 2 * w.b.heads + (int64_t)(w.keys / kGradTile) * 4 * kv_heads;
+  for (int64_t r = 0; r < w.b.total_q; r += w.rows) {
+    w.r_begin = (int32_t)r;
+    hipLaunchKernelGGL(bwd_wide_ds_kernel, dim3((unsigned)ds_items), dim3(kWideThreads), 0, stream, w);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(bwd_wide_grad_kernel, dim3((unsigned)grad_items), dim3(kWideThreads), 0, stream, w);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+}  // namespace karpo

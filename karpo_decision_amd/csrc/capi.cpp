@@ -349,6 +349,55 @@ BwdSizes bwd_sizes_of(const KarpoAttnBwdArgs* b) {
   return z;
 }
 
+// Head size 512, one sequence without a left bound or spans: the chunked path (attn_bwd_wide.hip) and the workspace
+// that it takes past the statistics (P and dS of a chunk of query rows; with more than one chunk, dK and dV in fp32).
+// rows 0: not for this call.
+struct WideSizes {
+  int64_t rows, keys, p_offset, ds_offset, acc_offset, bytes;
+};
+
+constexpr int64_t kWideBytes = (int64_t)4 << 30;  // P and dS of one chunk at most
+constexpr int64_t kWideTile = 256;
+
+// The largest chunks that `limit` bytes of workspace hold (SIZE_MAX: the path's own choice).
+WideSizes wide_sizes_of(const KarpoAttnBwdArgs* b, const BwdSizes& z, size_t limit) {
+  const KarpoAttnArgs* a = &b->fwd;
+  WideSizes w = {0, 0, 0, 0, 0, 0};
+  if (a->head_dim != 512 || a->n_seq != 1 || a->n_spans != 0 || a->window_left >= 0 || a->total_q < 1 ||
+      a->total_k < 1 || a->total_q > INT32_MAX - kWideTile || a->total_k > INT32_MAX - kWideTile)
+    return w;
+  const int64_t keys = (a->total_k + kWideTile - 1) / kWideTile * kWideTile;
+  const int64_t all = (a->total_q + kWideTile - 1) / kWideTile * kWideTile;
+  const int64_t row = 2 * 2 * keys * a->heads;                  // bytes of P and dS per query row
+  const int64_t kept = 2 * keys * a->kv_heads * 512 * 4;        // dK and dV in fp32, with more than one chunk
+  const int64_t room = (limit > (size_t)INT64_MAX ? INT64_MAX : (int64_t)limit) - z.stats_bytes;
+  int64_t chunks = 1;
+  if (row * all > ka_min(kWideBytes, room)) {
+    const int64_t most = ka_min(kWideBytes, room - kept) / row / kWideTile * kWideTile;
+    if (most < kWideTile) return w;
+    chunks = (all + most - 1) / most;
+  }
+  const int64_t rows = ((all + chunks - 1) / chunks + kWideTile - 1) / kWideTile * kWideTile;
+  if ((rows / 256) * (keys / 128) * a->heads > INT32_MAX ||
+      (rows / 256) * 2 * a->heads + (keys / 256) * 4 * a->kv_heads > INT32_MAX)
+    return w;
+  w.rows = rows;
+  w.keys = keys;
+  w.p_offset = z.stats_bytes;
+  w.ds_offset = w.p_offset + row / 2 * rows;
+  w.acc_offset = w.ds_offset + row / 2 * rows;
+  w.bytes = w.acc_offset + (chunks > 1 ? kept : 0);
+  return w;
+}
+
+// The chunked path addresses a tile's 256 rows with 32-bit byte offsets.
+bool wide_strides(const KarpoAttnBwdArgs* b) {
+  const int64_t strides[] = {b->fwd.q_stride_tok, b->fwd.k_stride_tok, b->fwd.v_stride_tok, b->d_o_stride_tok};
+  for (int64_t s : strides)
+    if ((s + 512) * kWideTile * 2 >= (int64_t)INT32_MAX) return false;
+  return true;
+}
+
 int check_bwd(const KarpoAttnBwdArgs* b) {
   if (b == nullptr) return KARPO_ATTN_ERR_NULL;
   const KarpoAttnArgs* a = &b->fwd;
@@ -365,6 +414,16 @@ extern "C" int karpo_attn_bwd_workspace_bytes(const KarpoAttnBwdArgs* b, size_t*
   if (st != KARPO_ATTN_OK) return st;
   if (bytes == nullptr) return KARPO_ATTN_ERR_NULL;
   *bytes = (size_t)bwd_sizes_of(b).bytes;
+  return KARPO_ATTN_OK;
+}
+
+extern "C" int karpo_attn_bwd_workspace_best_bytes(const KarpoAttnBwdArgs* b, size_t* bytes) {
+  const int st = check_bwd(b);
+  if (st != KARPO_ATTN_OK) return st;
+  if (bytes == nullptr) return KARPO_ATTN_ERR_NULL;
+  const BwdSizes z = bwd_sizes_of(b);
+  const WideSizes w = wide_sizes_of(b, z, SIZE_MAX);
+  *bytes = (size_t)(w.rows > 0 && wide_strides(b) && w.bytes > z.bytes ? w.bytes : z.bytes);
   return KARPO_ATTN_OK;
 }
 
@@ -452,6 +511,21 @@ extern "C" int karpo_attn_bwd(const KarpoAttnBwdArgs* b, void* stream) {
   p.scale = a->scale;
   p.partial = reinterpret_cast<float*>(ws + z.partial_offset);
   p.slots = (int32_t)split_slots(gk);
+  const WideSizes wide = wide_sizes_of(b, z, a->workspace_bytes);
+  if (wide.rows > 0 && wide_strides(b)) {
+    BwdWideParams w;
+    w.b = p;
+    w.p = reinterpret_cast<uint16_t*>(ws + wide.p_offset);
+    w.ds = reinterpret_cast<uint16_t*>(ws + wide.ds_offset);
+    w.acc = reinterpret_cast<float*>(ws + wide.acc_offset);
+    w.total_k = (int32_t)a->total_k;
+    w.rows = (int32_t)wide.rows;
+    w.keys = (int32_t)wide.keys;
+    w.r_begin = 0;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (launch_bwd_stats(p, s) != hipSuccess || launch_bwd_wide(w, s) != hipSuccess) return KARPO_ATTN_ERR_LAUNCH;
+    return KARPO_ATTN_OK;
+  }
   int32_t* const tile_base = ints + z.tile_bases;
   if (launch_bwd(p, a->head_dim, gq, gk, ints + z.plan_q, ints + z.plan_k, z.tiles_q, z.items_k, (int)z.tiles_q, 0,
                  (int)z.tiles_k, (int)z.merges_k, tile_base, tile_base + a->n_seq + 1, a->n_seq,

@@ -75,6 +75,22 @@ struct BwdParams {
 // Head size 512: the dQ and dK / dV kernels of wave pairs (attn_bwd_pair.hip), after the statistics pass.
 hipError_t launch_bwd_pair(const BwdParams& p, const Geometry& gq, const Geometry& gk, int32_t* plan_q,
                            int32_t* plan_k, int64_t items_q, int64_t items_k, hipStream_t stream);
+// Each row's log2-domain LSE and -rowsum(dO * O) into p.stats, in a pass of its own (head size 512).
+hipError_t launch_bwd_stats(const BwdParams& p, hipStream_t stream);
+
+// Head size 512, one sequence, no left bound and no spans (attn_bwd_wide.hip): P and dS of `rows` query rows at a time
+// in the workspace. The statistics pass runs before it.
+struct BwdWideParams {
+  BwdParams b;
+  uint16_t* p;   // [heads][keys / 16][rows / 8][16 keys, swizzled][8 rows] bf16
+  uint16_t* ds;  // the same for dS
+  float* acc;    // dK and dV between chunks of rows, fp32 [keys / 256][2][kv heads][2][256 x 256], in register order
+  int32_t total_k;
+  int32_t rows;     // query rows per chunk, a multiple of 256
+  int32_t keys;     // total_k rounded up to 256
+  int32_t r_begin;  // the chunk's first query row (set by the launch)
+};
+hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream);
 // items_q / items_k: the work lists' item capacities (the grids), tiles_q / tiles_k their tile capacities, merges_k
 // the key tiles' split capacity.
 hipError_t launch_bwd(const BwdParams& p, int head_dim, const Geometry& gq, const Geometry& gk, int32_t* plan_q,

@@ -313,6 +313,58 @@ def test_head_512_one_sequence_cases_of_the_reference(gpu, causal):
             assert r < REL_FRO, ((lq, lk), name, r)
 
 
+@pytest.mark.parametrize("lq,lk,pad,heads,kv_heads,right", [
+    (1, 1, 3, 8, 4, 0),        # one row
+    (256, 256, 0, 8, 1, 0),    # exactly one tile
+    (513, 1000, 0, 16, 2, 0),  # one row past two tiles, keys not a multiple of a tile, Lk > Lq
+    (700, 333, 5, 8, 8, 0),    # Lq > Lk: rows and key tiles that see nothing
+    (400, 900, 0, 6, 3, -1),   # bidirectional, a head count that does not spread over the XCDs
+    (1030, 1030, 90, 8, 1, 70),  # keys ahead of the diagonal
+])
+def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, kv_heads, right):
+    """One sequence at head size 512: the path that keeps P and dS of a chunk of query rows in the workspace, in one
+    chunk and in chunks of 256 rows (the workspace that leaves room for no more), against the oracle's float32
+    gradients and the wave-pair kernels (which the least workspace selects). The workspace and the rows past the
+    sequence hold NaN, which reach no gradient. Both paths round P and dS to bf16 and sum in fp32, so each is within
+    REL_FRO of float32, and they differ only by the order of their fp32 sums: a rounding of P, dS or a result to bf16
+    may then fall the other way in a few elements, 2^-9 at most each, so below 2^-10 over the norm. (One key: dS is a
+    difference that cancels, only dV is compared.)"""
+    import ctypes
+
+    dev = torch.device("cuda")
+    q, k, v, do, _, _, _ = make_pack([lq + pad], [lk + pad], heads, kv_heads, 512, seed=lq)
+    want = oa.packed_grads(q[:lq], k[:lk], v[:lk], do[:lq], [0, lq], [0, lk], 0.05, -1, right, dtype=torch.float32)[1:]
+    for t, n in ((q, lq), (k, lk), (v, lk), (do, lq)):
+        t[n:] = float("nan")
+    q, k, v, do = (t.to(dev) for t in (q, k, v, do))
+    qc, kc = (torch.tensor([0, n], dtype=torch.int32, device=dev) for n in (lq, lk))
+    out, lse = ops.packed_attention_lse(q, k, v, qc, kc, lq, 0.05, -1, right, None)
+    keys = -(-(lk + pad) // 256) * 256
+    # statistics, P and dS of 256 rows, dK and dV in fp32
+    chunk = -(-heads * 2 * (lq + pad) * 4 // 256) * 256 + 4 * 256 * keys * heads + 2 * keys * kv_heads * 512 * 4
+    got = {}
+    for form in ("least", "chunks", "best"):
+        def workspace(lib, fn, args, device):
+            least, best = ctypes.c_size_t(), ctypes.c_size_t()
+            assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(args), ctypes.byref(least)) == 0
+            assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(args), ctypes.byref(best)) == 0
+            size = {"least": least.value, "chunks": max(least.value, chunk), "best": best.value}[form]
+            assert best.value >= size or form == "chunks"
+            return torch.full((size,), 255, dtype=torch.uint8, device=device)
+
+        monkeypatch.setattr(ops, "_workspace", workspace)
+        print("head 512 one sequence", (lq, lk), form, flush=True)
+        got[form] = ops.packed_attention_backward(do, q, k, v, out, lse, qc, kc, lq, 0.05, -1, right, None)
+        torch.cuda.synchronize()
+        for name, x, w, pair in zip(("dq", "dk", "dv"), got[form], want, got["least"]):
+            if lk == 1 and name != "dv":
+                continue
+            n = w.shape[0]
+            r, rp = rel(x[:n], w), rel(x[:n], pair[:n])
+            print("   ", name, f"rel {r:.2e}, against the pairs {rp:.2e}", flush=True)
+            assert r < REL_FRO and rp < 2.0 ** -10, (form, name, r, rp)
+
+
 def test_sliding_case_of_the_reference(gpu):
     """The reference's FA4 sliding test (tests/gpu/test_packed_gemma.py:70-104): head size 256, 32 / 16 heads, window
     1023, queries and keys with their own bounds (three branches after a shared tail), loss sum(out * linspace(-1, 1));
