@@ -18,12 +18,11 @@
 //   * bwd_dkdv_kernel (key-stationary, tiles of 128 keys, four waves of 32): K and V of the wave's keys in registers,
 //     the query rows that see the tile streamed in steps of 32 rows of one head (every head of the GQA group in turn,
 //     which sums the group's gradients): S = Q K^T and dP = dO V^T with Q and dO as row operands, dV^T += dO^T P and
-//     dK^T += Q^T dS with Q and dO read transposed from the same tiles (S layout; a dV-only launch stages dO in the
-//     transposed-read layout, whose copies read whole rows). One launch computes both (MODE 3; at head sizes 64 and
-//     256 one wave per SIMD holds both accumulators in 256 AGPRs);
+//     dK^T += Q^T dS with Q and dO read transposed from the same tiles (S layout), both in one launch (head sizes 64 and
+//     256: one wave per SIMD holds both accumulators in 256 AGPRs);
 //   * bwd_dkdv2_kernel (head size 128): both gradients in one launch at two waves per SIMD, eight waves per key tile
 //     in two groups that take alternate row steps, K and V in LDS instead of registers (30.7 -> 28.1 ms for the 32k
-//     layer's backward against dV and dK as two launches, MODE 1 and MODE 2, each recomputing S: KA_BWD2 0).
+//     layer's backward against dV and dK as two launches that each recomputed S).
 // Both streams advance their copy addresses by pointer increments per step (no per-step address recomputation: the
 // scalar unit is shared by the CU's waves and a step is short).
 // Rows of a product's row operand are fed in the order that swaps bits 2 and 3 of the row index (key_row), so each
@@ -42,18 +41,9 @@ namespace karpo {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
-// Key-tile workgroups from which head size 128 runs dK and dV as two launches.
-constexpr int64_t kSplitKeyTiles = 8 * kComputeUnits;
-// Head size 128 computes dK and dV in bwd_dkdv2_kernel; KA_BWD2 0 restores the two launches (large packs) or the
-// one-wave-per-SIMD MODE 3 launch (small packs), for A/B measurements.
-#ifndef KA_BWD2
-#define KA_BWD2 1
-#endif
-
 template <int D> struct BwdCfg {
   static constexpr int OCC_Q = D >= 256 ? 1 : 2;  // waves per SIMD the registers are budgeted for
   static constexpr int BLOCKS_Q = OCC_Q * 4 / bwd_q_waves(D) > 0 ? OCC_Q * 4 / bwd_q_waves(D) : 1;
-  template <int MODE> static constexpr int occ_k() { return MODE == 3 ? 1 : MODE == 1 ? 3 : 2; }
 };
 
 // Row (within a 32-row step) of result register j of a lane in half `half` (row operands fed in key_row order).
@@ -212,14 +202,7 @@ __global__ __launch_bounds__(64 * bwd_q_waves(D), BwdCfg<D>::BLOCKS_Q) void bwd_
   // copies: K and V in the S layout (zeros past the sequence's last key)
   const uint16_t* kbase = p.k + (int64_t)kvh * p.sk_h + (int64_t)ka * p.sk_t;
   const uint16_t* vbase = p.v + (int64_t)kvh * p.sv_h + (int64_t)ka * p.sv_t;
-  uint32_t kk_off[INSTS], vk_off[INSTS];
-#pragma unroll
-  for (int r = 0; r < INSTS; ++r) {
-    int key, colm;
-    s_dma_source<D>(wave * INSTS + r, lane, &key, &colm);
-    kk_off[r] = (uint32_t)(key * p.sk_t + colm) * 2u;
-    vk_off[r] = (uint32_t)(key * p.sv_t + colm) * 2u;
-  }
+  const uint32_t kk_off = s_block_base<D, INSTS>(wave, lane, p.sk_t), vk_off = s_block_base<D, INSTS>(wave, lane, p.sv_t);
   const uint16_t* c_k = kbase + (int64_t)j_first * p.sk_t;
   const uint16_t* c_v = vbase + (int64_t)j_first * p.sv_t;
   const int64_t k_step = (int64_t)BN * p.sk_t, v_step = (int64_t)BN * p.sv_t;
@@ -233,8 +216,8 @@ __global__ __launch_bounds__(64 * bwd_q_waves(D), BwdCfg<D>::BLOCKS_Q) void bwd_
     for (int r = 0; r < INSTS; ++r)
       if (BLKS % W == 0 || wave * INSTS + r < BLKS) {
         const int at = (wave * INSTS + r) * 1024;
-        dma_16b(ks, rows * (int)p.sk_t * 2, tkk + at, kk_off[r]);
-        dma_16b(vs, rows * (int)p.sv_t * 2, tvk + at, vk_off[r]);
+        dma_16b(ks, rows * (int)p.sk_t * 2, tkk + at, s_block(kk_off, r));
+        dma_16b(vs, rows * (int)p.sv_t * 2, tvk + at, s_block(vk_off, r));
       }
   };
   // row reads of chunk 2 dc + half: k_read[dc & 1] + (dc >> 1) * 1024; transposed reads: t_read[rr] + kc, db offsets
@@ -386,21 +369,22 @@ __device__ __forceinline__ KeyRows key_rows_seen(const BwdParams& p, int key, bo
   return r;
 }
 
-// ---- dK, dV: key tiles of 128 (plan items of the bounds swapped: segment, key tile), 32 keys per wave. MODE bit 0:
-// compute dV, bit 1: dK.
-template <int D, int MODE>
-__global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) void bwd_dkdv_kernel(BwdParams p) {
-  constexpr bool DV = (MODE & 1) != 0, DK = (MODE & 2) != 0;
+// ---- dK, dV: key tiles of 128 (plan items of the bounds swapped: segment, key tile), 32 keys per wave,
+// both gradients, one wave per SIMD (head sizes 64 and 256).
+template <int D>
+__global__ __launch_bounds__(64 * kBwdWaves, 1) void bwd_dkdv_kernel(BwdParams p) {
   constexpr int W = kBwdWaves, BQ = kBwdStep;
   constexpr int DC = D / 16, DB = D / 32, KC = BQ / 16;
   constexpr int TILE = BQ * D * 2, BLKS = TILE / 1024, INSTS = (BLKS + W - 1) / W;
   __shared__ __attribute__((aligned(1024))) char qk0[TILE];  // Q (S layout: rows for S, transposed for dK)
   __shared__ __attribute__((aligned(1024))) char qk1[TILE];
-  __shared__ __attribute__((aligned(1024))) char ok0[TILE];  // dO (S layout: rows for dP, transposed for dV; dV alone: transposed-read layout)
+  __shared__ __attribute__((aligned(1024))) char ok0[TILE];  // dO (S layout: rows for dP, transposed for dV)
   __shared__ __attribute__((aligned(1024))) char ok1[TILE];
   __shared__ __attribute__((aligned(256))) float sts0[2 * BQ];  // log2 LSE, then -D, of the step's rows
   __shared__ __attribute__((aligned(256))) float sts1[2 * BQ];
   __shared__ int red[2][W];
+  __shared__ __attribute__((aligned(16))) int32_t seen_s[64 * W][4];  // the lanes' row ranges, for the masked steps: four
+                                                                      // registers less (at head size 256 they spilled)
 
   if (p.plan[2] != BQ || p.plan[5] != W) return;
   const int item = blockIdx.x / p.n_hg;
@@ -423,7 +407,10 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
   const int key = ktile * keys_per_tile + wave * 32 + col;
   const bool valid = key < lk;
   const KeyRows seen = key_rows_seen(p, key, valid, qa, lq, delta);
-  const int rlo = seen.lo, rhi = seen.hi, srl = seen.sl, srh = seen.sh;
+  seen_s[tid][0] = seen.lo;
+  seen_s[tid][1] = seen.hi;
+  seen_s[tid][2] = seen.sl;
+  seen_s[tid][3] = seen.sh;
   const int wlo = seen.wlo, whi = seen.whi, wflo = seen.wflo, wfhi = seen.wfhi;
   if (lane == 0) {
     red[0][wave] = wlo;
@@ -439,10 +426,10 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
       u32x4 x = {0, 0, 0, 0}, y = {0, 0, 0, 0};
       if (valid) {
         x = *(const u32x4*)(kp + dc * 16);
-        if constexpr (DK) y = *(const u32x4*)(vp + dc * 16);
+        y = *(const u32x4*)(vp + dc * 16);
       }
       kop[dc] = __builtin_bit_cast(bf16x8, x);
-      if constexpr (DK) vop[dc] = __builtin_bit_cast(bf16x8, y);
+      vop[dc] = __builtin_bit_cast(bf16x8, y);
     }
   }
   __syncthreads();
@@ -461,18 +448,7 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
   const int s_begin = parts > 1 ? (int)((int64_t)part * all_steps / parts) : 0;
   const int n_steps = parts > 1 ? (int)((int64_t)(part + 1) * all_steps / parts) - s_begin : all_steps;
 
-  // dV alone reads dO only transposed: it keeps the transposed-read layout, whose copy reads whole rows (the S
-  // layout's reads 64 bytes of each of 16 rows per instruction)
-  constexpr bool OV = MODE == 1;
-  uint32_t qk_off[INSTS], ok_off[INSTS];
-#pragma unroll
-  for (int r = 0; r < INSTS; ++r) {
-    int row, colm;
-    s_dma_source<D>(wave * INSTS + r, lane, &row, &colm);
-    qk_off[r] = (uint32_t)(row * p.sq_t + colm) * 2u;
-    if constexpr (OV) v_dma_source<D>(wave * INSTS + r, lane, &row, &colm);
-    ok_off[r] = (uint32_t)(row * p.sdo_t + colm) * 2u;
-  }
+  const uint32_t qk_off = s_block_base<D, INSTS>(wave, lane, p.sq_t), ok_off = s_block_base<D, INSTS>(wave, lane, p.sdo_t);
   // Steps visit the row steps of head kvh * group from the last (r_last) down to r_first, then the group's next
   // head's. Downwards: under a causal mask every key tile's rows end at the sequence's end, so the tiles that run at
   // once read the same Q / dO rows at about the same time (L2 hits) instead of rows a tile apart. The copy cursor
@@ -507,8 +483,8 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
     for (int r = 0; r < INSTS; ++r)
       if (BLKS % W == 0 || wave * INSTS + r < BLKS) {
         const int at = (wave * INSTS + r) * 1024;
-        dma_16b(qs, rows * (int)p.sq_t * 2, tqk + at, qk_off[r]);
-        dma_16b(os, rows * (int)p.sdo_t * 2, tok + at, ok_off[r]);
+        dma_16b(qs, rows * (int)p.sq_t * 2, tqk + at, s_block(qk_off, r));
+        dma_16b(os, rows * (int)p.sdo_t * 2, tok + at, s_block(ok_off, r));
       }
     if (wave == W - 1) {  // 32 log2 LSE (lanes 0-31) then 32 -D (lanes 32-63), 4 B per lane; zeros past the stats
       const __amdgpu_buffer_rsrc_t rs =
@@ -520,8 +496,6 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
   // row reads of chunk 2 dc + half: q_read[dc & 1] + (dc >> 1) * 1024; transposed reads: t_read[rr] + kc, db offsets
   const int q_read[2] = {s_offset<D>(key_row(col), half), s_offset<D>(key_row(col), 2 + half)};
   const int t_read[2] = {s_tr_base(lane, 0), s_tr_base(lane, 1)};
-  const int g = lane >> 4, jl = lane & 15;
-  const int v_read = v_offset<D>(8 * (g >> 1) + (jl >> 2), 16 * (g & 1) + 4 * (jl & 3));
   f32x16 dk[DB], dv[DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db) {
@@ -549,22 +523,18 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
     if (r0 < whi && r0 + BQ > wlo) {
       // dP starts from -D of this lane's result rows (half*8 .. and 16 + half*8 ..): the MFMAs leave dP - D
       f32x16 st = f32x16{}, dpt = f32x16{};
-      if constexpr (DK) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const f32x4 nd = *(const KA_LDS f32x4*)(tst + BQ + (u >> 1) * 16 + half * 8 + (u & 1) * 4);
+      for (int u = 0; u < 4; ++u) {
+        const f32x4 nd = *(const KA_LDS f32x4*)(tst + BQ + (u >> 1) * 16 + half * 8 + (u & 1) * 4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) dpt[4 * u + e] = nd[e];
-        }
+        for (int e = 0; e < 4; ++e) dpt[4 * u + e] = nd[e];
       }
 #pragma unroll
       for (int dc = 0; dc < DC; ++dc) {
         const bf16x8 a = *(const KA_LDS bf16x8*)(tqk + q_read[dc & 1] + (dc >> 1) * 1024);
         st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, kop[dc], st, 0, 0, 0);
-        if constexpr (DK) {
-          const bf16x8 b = *(const KA_LDS bf16x8*)(tok + q_read[dc & 1] + (dc >> 1) * 1024);
-          dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, vop[dc], dpt, 0, 0, 0);
-        }
+        const bf16x8 b = *(const KA_LDS bf16x8*)(tok + q_read[dc & 1] + (dc >> 1) * 1024);
+        dpt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, vop[dc], dpt, 0, 0, 0);
       }
       // the step rows' log2 LSE for this lane's result registers
       f32x4 ls[4];
@@ -576,6 +546,7 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
 #pragma unroll
       for (int jj = 0; jj < 2 * KC * 4; ++jj) x[jj] = __builtin_fmaf(st[jj], c, -ls[jj >> 2][jj & 3]);
       if (!(r0 >= wflo && r0 + BQ <= wfhi)) {
+        const int rlo = seen_s[tid][0], rhi = seen_s[tid][1], srl = seen_s[tid][2], srh = seen_s[tid][3];
 #pragma unroll
         for (int jj = 0; jj < 2 * KC * 4; ++jj) {
           const int row = r0 + result_row(jj, half);
@@ -591,8 +562,8 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
         for (int t = 0; t < 8; ++t) {
           const int jj = kc * 8 + t;
           const float pr = __builtin_amdgcn_exp2f(x[jj]);
-          if constexpr (DV) pb[kc][t] = (__bf16)pr;
-          if constexpr (DK) dsb[kc][t] = (__bf16)(pr * dpt[jj]);
+          pb[kc][t] = (__bf16)pr;
+          dsb[kc][t] = (__bf16)(pr * dpt[jj]);
         }
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) {
@@ -602,20 +573,13 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
 #pragma unroll
           for (int rr = 0; rr < 2; ++rr) {
             const int at = t_read[rr] + kc * (D / 8) * 256 + db * 1024;
-            const int vt = OV ? v_read + (kc * 4 + rr) * (D / 16) * 128 + db * 256 : at;
-            if constexpr (DV)
-              ov[rr] = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(tok + vt)));
-            if constexpr (DK)
-              qv[rr] = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(tqk + at)));
+            ov[rr] = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(tok + at)));
+            qv[rr] = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(tqk + at)));
           }
-          if constexpr (DV) {
-            const bf16x8 ao = __builtin_shufflevector(ov[0], ov[1], 0, 1, 2, 3, 4, 5, 6, 7);
-            dv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ao, pb[kc], dv[db], 0, 0, 0);
-          }
-          if constexpr (DK) {
-            const bf16x8 aq = __builtin_shufflevector(qv[0], qv[1], 0, 1, 2, 3, 4, 5, 6, 7);
-            dk[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq, dsb[kc], dk[db], 0, 0, 0);
-          }
+          const bf16x8 ao = __builtin_shufflevector(ov[0], ov[1], 0, 1, 2, 3, 4, 5, 6, 7);
+          dv[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ao, pb[kc], dv[db], 0, 0, 0);
+          const bf16x8 aq = __builtin_shufflevector(qv[0], qv[1], 0, 1, 2, 3, 4, 5, 6, 7);
+          dk[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq, dsb[kc], dk[db], 0, 0, 0);
         }
       }
     }
@@ -636,12 +600,10 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        if constexpr (DK)
-          *(float4*)(base + db * 32 + g4 * 8) = float4{dk[db][g4 * 4], dk[db][g4 * 4 + 1], dk[db][g4 * 4 + 2],
-                                                       dk[db][g4 * 4 + 3]};
-        if constexpr (DV)
-          *(float4*)(base + KT * D + db * 32 + g4 * 8) = float4{dv[db][g4 * 4], dv[db][g4 * 4 + 1],
-                                                                dv[db][g4 * 4 + 2], dv[db][g4 * 4 + 3]};
+        *(float4*)(base + db * 32 + g4 * 8) = float4{dk[db][g4 * 4], dk[db][g4 * 4 + 1], dk[db][g4 * 4 + 2],
+                                                     dk[db][g4 * 4 + 3]};
+        *(float4*)(base + KT * D + db * 32 + g4 * 8) = float4{dv[db][g4 * 4], dv[db][g4 * 4 + 1],
+                                                              dv[db][g4 * 4 + 2], dv[db][g4 * 4 + 3]};
       }
     return;
   }
@@ -652,18 +614,14 @@ __global__ __launch_bounds__(64 * kBwdWaves, BwdCfg<D>::template occ_k<MODE>()) 
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int g4 = 0; g4 < 4; ++g4) {
-        if constexpr (DK) {
-          u32x2 a;
-          a[0] = pack_bf16(dk[db][g4 * 4] * p.scale, dk[db][g4 * 4 + 1] * p.scale);
-          a[1] = pack_bf16(dk[db][g4 * 4 + 2] * p.scale, dk[db][g4 * 4 + 3] * p.scale);
-          *(u32x2*)(kq + db * 32 + g4 * 8) = a;
-        }
-        if constexpr (DV) {
-          u32x2 b;
-          b[0] = pack_bf16(dv[db][g4 * 4], dv[db][g4 * 4 + 1]);
-          b[1] = pack_bf16(dv[db][g4 * 4 + 2], dv[db][g4 * 4 + 3]);
-          *(u32x2*)(vq + db * 32 + g4 * 8) = b;
-        }
+        u32x2 a;
+        a[0] = pack_bf16(dk[db][g4 * 4] * p.scale, dk[db][g4 * 4 + 1] * p.scale);
+        a[1] = pack_bf16(dk[db][g4 * 4 + 2] * p.scale, dk[db][g4 * 4 + 3] * p.scale);
+        *(u32x2*)(kq + db * 32 + g4 * 8) = a;
+        u32x2 b;
+        b[0] = pack_bf16(dv[db][g4 * 4], dv[db][g4 * 4 + 1]);
+        b[1] = pack_bf16(dv[db][g4 * 4 + 2], dv[db][g4 * 4 + 3]);
+        *(u32x2*)(vq + db * 32 + g4 * 8) = b;
       }
   }
 }
@@ -754,14 +712,7 @@ __global__ __launch_bounds__(64 * 2 * kBwdWaves, 2) void bwd_dkdv2_kernel(BwdPar
   const int n_iter = (n_steps + 1) / 2;
 
   const int gofs = rs * TILE;  // this group's buffers in the two-group arrays
-  uint32_t qk_off[INSTS], ok_off[INSTS];
-#pragma unroll
-  for (int r = 0; r < INSTS; ++r) {
-    int row, colm;
-    s_dma_source<D>(kw * INSTS + r, lane, &row, &colm);
-    qk_off[r] = (uint32_t)(row * p.sq_t + colm) * 2u;
-    ok_off[r] = (uint32_t)(row * p.sdo_t + colm) * 2u;
-  }
+  const uint32_t qk_off = s_block_base<D, INSTS>(kw, lane, p.sq_t), ok_off = s_block_base<D, INSTS>(kw, lane, p.sdo_t);
   // the steps in bwd_dkdv_kernel's order (rows downwards, then the group's next head), each group taking every other
   const int r_last = r_first + (n_rsteps - 1) * BQ;
   const int h0 = kvh * p.group;
@@ -802,8 +753,8 @@ __global__ __launch_bounds__(64 * 2 * kBwdWaves, 2) void bwd_dkdv2_kernel(BwdPar
 #pragma unroll
     for (int r = 0; r < INSTS; ++r) {
       const int at = gofs + (kw * INSTS + r) * 1024;
-      dma_16b(qs, rows * (int)p.sq_t * 2, tqk + at, qk_off[r]);
-      dma_16b(os, rows * (int)p.sdo_t * 2, tok + at, ok_off[r]);
+      dma_16b(qs, rows * (int)p.sq_t * 2, tqk + at, s_block(qk_off, r));
+      dma_16b(os, rows * (int)p.sdo_t * 2, tok + at, s_block(ok_off, r));
     }
     if (kw == KW - 1) {  // 32 log2 LSE (lanes 0-31) then 32 -D (lanes 32-63), 4 B per lane; zeros past the stats
       const __amdgpu_buffer_rsrc_t rsrc =
@@ -1027,7 +978,7 @@ __global__ __launch_bounds__(kBwdMergeThreads) void bwd_merge_kernel(BwdParams p
 
 template <int D>
 static hipError_t launch_bwd_d(const BwdParams& p, const Geometry& gq, const Geometry& gk, int32_t* plan_q,
-                               int32_t* plan_k, int64_t items_q, int64_t items_k, int64_t tiles_k, int merges_k,
+                               int32_t* plan_k, int64_t items_q, int64_t items_k, int merges_k,
                                hipStream_t stream) {
   // the rows' statistics come from the dQ kernel (no separate pass below head size 512)
   hipError_t e;
@@ -1046,16 +997,8 @@ static hipError_t launch_bwd_d(const BwdParams& p, const Geometry& gq, const Geo
   pk.n_hg = gk.n_hg;
   const dim3 grid((unsigned)(items_k * gk.n_hg));
   if (items_k > 0) {
-    if (D == 128 && KA_BWD2) {
-      if constexpr (D == 128) hipLaunchKernelGGL(bwd_dkdv2_kernel<D>, grid, dim3(2 * 64 * kBwdWaves), 0, stream, pk);
-    } else if (D == 128 && tiles_k * gk.n_hg >= kSplitKeyTiles) {
-      if constexpr (D == 128) {
-        hipLaunchKernelGGL((bwd_dkdv_kernel<D, 1>), grid, dim3(64 * kBwdWaves), 0, stream, pk);
-        hipLaunchKernelGGL((bwd_dkdv_kernel<D, 2>), grid, dim3(64 * kBwdWaves), 0, stream, pk);
-      }
-    } else {
-      hipLaunchKernelGGL((bwd_dkdv_kernel<D, 3>), grid, dim3(64 * kBwdWaves), 0, stream, pk);
-    }
+    if constexpr (D == 128) hipLaunchKernelGGL(bwd_dkdv2_kernel<D>, grid, dim3(2 * 64 * kBwdWaves), 0, stream, pk);
+    else hipLaunchKernelGGL(bwd_dkdv_kernel<D>, grid, dim3(64 * kBwdWaves), 0, stream, pk);
   }
   e = hipGetLastError();
   if (D > 128 || e != hipSuccess || items_k <= 0 || merges_k <= 0) return e;
@@ -1083,9 +1026,9 @@ hipError_t launch_bwd(const BwdParams& p, int head_dim, const Geometry& gq, cons
   hipError_t e = launch_plan(jobs, 2, n_seq, stream);
   if (e != hipSuccess) return e;
   switch (head_dim) {
-    case 64: return launch_bwd_d<64>(p, gq, gk, plan_q, plan_k, items_q, items_k, tiles_k, merges_k, stream);
-    case 128: return launch_bwd_d<128>(p, gq, gk, plan_q, plan_k, items_q, items_k, tiles_k, merges_k, stream);
-    case 256: return launch_bwd_d<256>(p, gq, gk, plan_q, plan_k, items_q, items_k, tiles_k, merges_k, stream);
+    case 64: return launch_bwd_d<64>(p, gq, gk, plan_q, plan_k, items_q, items_k, merges_k, stream);
+    case 128: return launch_bwd_d<128>(p, gq, gk, plan_q, plan_k, items_q, items_k, merges_k, stream);
+    case 256: return launch_bwd_d<256>(p, gq, gk, plan_q, plan_k, items_q, items_k, merges_k, stream);
     case 512:
       e = launch_bwd_stats(p, stream);
       return e != hipSuccess ? e : launch_bwd_pair(p, gq, gk, plan_q, plan_k, items_q, items_k, stream);

@@ -28,16 +28,6 @@ namespace karpo {
 constexpr int kPairWaves = 4;  // two pairs per workgroup
 constexpr int kPairStep = 32;  // keys (dQ) or query rows (dK, dV) per step
 
-// A wave's eight 1 KiB copy blocks per tile (blocks 8w .. 8w+7 of 32) at head size 512, as byte offsets from the
-// tile's first row (s_dma_source of block 8w + r): they advance 64 B per block, so one register per tile holds them
-// instead of eight (checked against the per-block formula for every wave, lane and block).
-__device__ __forceinline__ uint32_t s_block_base(int wave, int lane, int64_t stride) {
-  int row, colm;
-  s_dma_source<512>(wave * 8, lane, &row, &colm);
-  return (uint32_t)(row * stride + colm) * 2u;
-}
-__device__ __forceinline__ uint32_t s_block(uint32_t base, int r) { return base + (uint32_t)r * 64u; }
-
 // The pair's partial S (q4 0-3) and dP (q4 4-7) of one wave: 32 floats per lane as 8 f32x4 [q4][lane].
 __device__ __forceinline__ void exchange_write(KA_LDS f32x4* slot, int lane, const f32x16& a, const f32x16& b,
                                                bool with_b) {
@@ -134,7 +124,7 @@ __global__ __launch_bounds__(64 * kPairWaves, 1) void bwd_dq_pair_kernel(BwdPara
   const int n_steps = klo < khi ? (khi - j_first + BN - 1) / BN : 0;
 
   static_assert(D == 512 && INSTS == 8, "the block offsets below are those of head size 512");
-  const uint32_t k_off = s_block_base(wave, lane, p.sk_t), v_off = s_block_base(wave, lane, p.sv_t);
+  const uint32_t k_off = s_block_base<D, INSTS>(wave, lane, p.sk_t), v_off = s_block_base<D, INSTS>(wave, lane, p.sv_t);
   KA_LDS char* const k0 = (KA_LDS char*)k0_s;
   KA_LDS char* const k1 = (KA_LDS char*)k1_s;
   KA_LDS char* const vt = (KA_LDS char*)v_s;
@@ -332,7 +322,7 @@ __global__ __launch_bounds__(64 * kPairWaves, 1) void bwd_dkdv_pair_kernel(BwdPa
   const int n_steps = n_rsteps * p.group;
 
   static_assert(D == 512 && INSTS == 8, "the block offsets below are those of head size 512");
-  const uint32_t q_off = s_block_base(wave, lane, p.sq_t), o_off = s_block_base(wave, lane, p.sdo_t);
+  const uint32_t q_off = s_block_base<D, INSTS>(wave, lane, p.sq_t), o_off = s_block_base<D, INSTS>(wave, lane, p.sdo_t);
   KA_LDS char* const q0 = (KA_LDS char*)q0_s;
   KA_LDS char* const q1 = (KA_LDS char*)q1_s;
   KA_LDS char* const o0 = (KA_LDS char*)o0_s;

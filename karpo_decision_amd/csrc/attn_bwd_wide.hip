@@ -9,12 +9,12 @@
 // 5,120 FLOPs need them, so keeping them takes less time than either the recomputation or the exchange: five products,
 // each a plain tiled matrix product with every accumulator in one wave's registers. Measured against the wave pairs
 // (32 / 4 heads, causal, MI355X): 497 -> 140 us at 512 rows, 2.09 -> 0.83 ms at 2,048, 12.4 -> 8.0 ms at 8,192, 48.1 ->
-// 29.9 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
+// 26.2 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
 // call takes this path when the workspace has room for a chunk of 256 rows.
 //
 // P and dS in the workspace: per head [key block of 16][chunk of 8 rows][16 keys][8 rows] bf16, the 16 keys of a
-// 256-byte run XOR-swizzled by the chunk index as in the S layout (mfma_common.h): the layout in which a tile is read
-// from LDS, so a copy instruction moves 1 KiB of consecutive bytes. A lane of kernel 1 holds one key's scores of 8
+// 256-byte run XOR-swizzled by the chunk index (key ^ 4 (chunk % 4): free of bank conflicts read either way), the layout
+// in which a tile is read from LDS: a copy instruction moves 1 KiB of consecutive bytes. A lane of kernel 1 holds one key's scores of 8
 // consecutive rows (the MFMA's A rows are taken in key_row order) and stores them as one 16-byte chunk; dK and dV read
 // those chunks directly as MFMA operands, dQ reads the same tile transposed.
 //
@@ -36,8 +36,9 @@ namespace karpo {
 constexpr int kWideD = 512;
 constexpr int kWideThreads = 512;               // eight waves
 constexpr int kDsRows = 256, kDsKeys = 128;     // kernel 1's tile
-constexpr int kDsStep = 64;                     // elements of D per step
-constexpr int kGradTile = 256, kGradStep = 64;  // kernel 2's outputs (both ways) and contraction step
+constexpr int kDsStep = 32;                     // elements of D per step
+constexpr int kGradTile = 256, kGradStep = 32;  // kernel 2's outputs (both ways) and contraction step
+constexpr int kRing = 4;                        // buffers: three steps of copies in flight
 
 // The sequence's bounds, clamped to the call's rows.
 struct WideSeq {
@@ -56,6 +57,13 @@ struct WideSeq {
   }
 };
 
+// Transposed read of a P or dS tile (chunks as columns): the lane's address in its first 16 keys and 32 rows.
+__device__ __forceinline__ int x_tr_base(int lane, int rr) {
+  const int g = lane >> 4, jl = lane & 15;
+  const int c = 2 * (g & 1) + ((jl >> 1) & 1);
+  return c * 256 + (((4 * rr + 8 * (g >> 1) + (jl >> 2)) ^ (c << 2)) * 16) + (jl & 1) * 8;
+}
+
 // Work index -> head with XCD w % 8 given heads that are neighbours (the same key/value head) where the count allows.
 __device__ __forceinline__ int spread_head(int i, int n) { return n % 8 == 0 ? (i % 8) * (n / 8) + i / 8 : i; }
 
@@ -63,37 +71,190 @@ __device__ __forceinline__ int spread_head(int i, int n) { return n % 8 == 0 ? (
 // flight): the copies a step needs are waited for by count.
 __device__ __forceinline__ void step_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// ---- kernel 1: P and dS of 256 rows x 128 keys of one head (eight waves of 64 x 64)
+// ---- kernel 1: P and dS of 256 rows x 128 keys of one head (eight waves of 64 x 64), for a run of key tiles: the next
+// tile's first copies are in flight while this one's P and dS are formed and stored, and a tile's exponentials run
+// beside its dP products
 __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_ds_kernel(BwdWideParams w) {
   constexpr int STEPS = kWideD / kDsStep;  // per product
+  constexpr int ALL = 2 * STEPS;           // S, then dP
+  static_assert(ALL % kRing == 0 && STEPS == 16, "a tile starts in buffer 0; four exponentials per dP step");
   constexpr int AT = kDsRows * kDsStep * 2, BT = kDsKeys * kDsStep * 2;
-  __shared__ __attribute__((aligned(1024))) char a0_s[AT], a1_s[AT], a2_s[AT];
-  __shared__ __attribute__((aligned(1024))) char b0_s[BT], b1_s[BT], b2_s[BT];
+  constexpr int COPIES = 3, STORES = 16;  // vector-memory operations of a wave per step and per tile's end
+  __shared__ __attribute__((aligned(1024))) char a0_s[AT], a1_s[AT], a2_s[AT], a3_s[AT];
+  __shared__ __attribute__((aligned(1024))) char b0_s[BT], b1_s[BT], b2_s[BT], b3_s[BT];
   __shared__ __attribute__((aligned(16))) float st_s[2][kDsRows];  // the rows' log2 LSE and -D
 
   const BwdParams& p = w.b;
   const WideSeq s(w);
-  const int key_tiles = w.keys / kDsKeys;
+  const int key_tiles = w.keys / kDsKeys, runs = (key_tiles + w.run - 1) / w.run;
   const int head = spread_head(blockIdx.x % p.heads, p.heads);
   const int rest = blockIdx.x / p.heads;
-  const int rt = rest / key_tiles, kt = rest - rt * key_tiles;
-  const int r0 = w.r_begin + rt * kDsRows, k0 = kt * kDsKeys;
-  const int k_pair = k0 & ~(kGradTile - 1);  // kernel 2 reads keys in tiles of 256
-  if (r0 >= s.lq || k_pair >= s.lk || r0 + kDsRows <= s.first_row(p.right, k_pair)) return;
+  const int rt = rest / runs;
+  const int r0 = w.r_begin + rt * kDsRows;
+  int kt = (rest - rt * runs) * w.run;
+  // the tiles that kernel 2 reads (keys in tiles of 256), and of those the ones that a row of this tile sees
+  if (r0 >= s.lq) return;
+  const int top = (int)min((int64_t)r0 + kDsRows - 1 + (s.lk - s.lq) + (p.right < 0 ? 0 : p.right), (int64_t)s.lk - 1);
+  const int seen = p.right < 0 ? s.lk : top + 1;  // keys
+  const int last = min((seen + kDsKeys - 1) / kDsKeys, kt + w.run);
+  const int read = min((seen + kGradTile - 1) / kGradTile * (kGradTile / kDsKeys), kt + w.run);
+  if (seen <= 0 || kt >= read) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
   const int wr = wave >> 1, wc = wave & 1;
-  // this lane's chunk (rows rt*256 + wr*64 + rb*32 + kc*16 + half*8 .. +8) of key k0 + wc*64 + cb*32 + col
+  // this lane's chunk (rows rt*256 + wr*64 + rb*32 + kc*16 + half*8 .. +8) of key kt*128 + wc*64 + cb*32 + col
   char* const out_p = (char*)(w.p + (int64_t)head * w.keys * w.rows);
   char* const out_s = (char*)(w.ds + (int64_t)head * w.keys * w.rows);
   const uint32_t run = (uint32_t)(w.rows / 8) * 256u;  // bytes per block of 16 keys
-  const uint32_t out_base =
-      (uint32_t)(kt * 8 + wc * 4 + (col >> 4)) * run + (uint32_t)(rt * 32 + wr * 8 + half) * 256u;
+  uint32_t out_base = (uint32_t)(kt * 8 + wc * 4 + (col >> 4)) * run + (uint32_t)(rt * 32 + wr * 8 + half) * 256u;
   const uint32_t out_key[2] = {(uint32_t)((col & 15) ^ (half << 2)) * 16u,
                                (uint32_t)((col & 15) ^ ((2 + half) << 2)) * 16u};
-  if (k0 >= s.lk || r0 + kDsRows <= s.first_row(p.right, k0)) {  // nothing seen, but read by kernel 2
+  if (kt < last) {
+    {
+      const int row = r0 + (tid & 255), which = tid >> 8;
+      st_s[which][tid & 255] = row < s.lq ? p.stats[((int64_t)head * 2 + which) * p.total_q + s.qa + row]
+                                          : (which ? 0.f : INFINITY);  // a row past the sequence has P = 0
+    }
+    const int kvh = head / p.group;
+    const uint16_t* const q = p.q + (int64_t)(s.qa + r0) * p.sq_t + (int64_t)head * p.sq_h;
+    const uint16_t* const o = p.dout + (int64_t)(s.qa + r0) * p.sdo_t + (int64_t)head * p.sdo_h;
+    const uint16_t* k = p.k + (int64_t)(s.ka + kt * kDsKeys) * p.sk_t + (int64_t)kvh * p.sk_h;
+    const uint16_t* v = p.v + (int64_t)(s.ka + kt * kDsKeys) * p.sv_t + (int64_t)kvh * p.sv_h;
+    const int64_t k_tile = (int64_t)kDsKeys * p.sk_t, v_tile = (int64_t)kDsKeys * p.sv_t;
+    const int rows = min(s.lq - r0, kDsRows);
+    // tiles in the S layout of 32 columns (16 rows x 64 B per copy): wave w copies A rows 32w .. +32, B rows 16w .. +16
+    int lrow, lcol;
+    s_dma_source<kDsStep>(0, lane, &lrow, &lcol);
+    const uint32_t q_off = (uint32_t)((wave * 32 + lrow) * (int)p.sq_t + lcol) * 2u;
+    const uint32_t o_off = (uint32_t)((wave * 32 + lrow) * (int)p.sdo_t + lcol) * 2u;
+    const uint32_t k_off = (uint32_t)((wave * 16 + lrow) * (int)p.sk_t + lcol) * 2u;
+    const uint32_t v_off = (uint32_t)((wave * 16 + lrow) * (int)p.sv_t + lcol) * 2u;
+    // step i of the tile at k, v (with `keys` of its keys in the sequence)
+    auto copy = [&](int i, const uint16_t* kb, const uint16_t* vb, int keys, KA_LDS char* a, KA_LDS char* b) {
+      const bool second = i >= STEPS;
+      const int at = (second ? i - STEPS : i) * kDsStep;
+      const int a_t = (int)(second ? p.sdo_t : p.sq_t) * 2, b_t = (int)(second ? p.sv_t : p.sk_t) * 2;
+      const uint32_t a_off = second ? o_off : q_off;
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+        dma_16b((second ? o : q) + at, rows * a_t, a + (wave * 2 + r) * 1024, a_off + (uint32_t)(r * 16 * a_t));
+      dma_16b((second ? vb : kb) + at, keys * b_t, b + wave * 1024, second ? v_off : k_off);
+    };
+    const int arow = key_row(col);
+    const int a_read[2] = {s_offset<kDsStep>(wr * 64 + arow, half), s_offset<kDsStep>(wr * 64 + arow, 2 + half)};
+    const int b_read[2] = {s_offset<kDsStep>(wc * 64 + col, half), s_offset<kDsStep>(wc * 64 + col, 2 + half)};
+    KA_LDS char* const at[kRing] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s, (KA_LDS char*)a2_s, (KA_LDS char*)a3_s};
+    KA_LDS char* const bt[kRing] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s, (KA_LDS char*)b2_s, (KA_LDS char*)b3_s};
+    const float c = p.c;
+
+    int keys = min(s.lk - kt * kDsKeys, kDsKeys);
+#pragma unroll
+    for (int i = 0; i < kRing - 1; ++i) copy(i, k, v, keys, at[i], bt[i]);
+    wait_vmcnt<2 * COPIES>();
+    step_barrier();
+    for (bool start = true;; start = false) {
+      const bool more = kt + 1 < last;
+      const int k0 = kt * kDsKeys, keys_next = min(s.lk - k0 - kDsKeys, kDsKeys);
+      f32x16 st[2][2], dp[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          st[i][j] = f32x16{};
+          dp[i][j] = f32x16{};
+        }
+#pragma unroll
+      for (int i = 0; i < ALL; ++i) {
+        constexpr int AHEAD = kRing - 1;
+        KA_LDS char* const an = at[(i + AHEAD) % kRing];
+        KA_LDS char* const bn = bt[(i + AHEAD) % kRing];
+        if (i + AHEAD < ALL) copy(i + AHEAD, k, v, keys, an, bn);
+        else if (more) copy(i + AHEAD - ALL, k + k_tile, v + v_tile, keys_next, an, bn);
+        __builtin_amdgcn_sched_barrier(0);  // the copies are issued first
+        const KA_LDS char* const a = at[i % kRing];
+        const KA_LDS char* const b = bt[i % kRing];
+#pragma unroll
+        for (int kk = 0; kk < kDsStep / 16; ++kk) {
+          bf16x8 x[2], y[2];
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            x[m] = *(const KA_LDS bf16x8*)(a + a_read[kk] + m * 2048);
+            y[m] = *(const KA_LDS bf16x8*)(b + b_read[kk] + m * 2048);
+          }
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+              f32x16& acc = i < STEPS ? st[m][n] : dp[m][n];
+              acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[m], y[n], acc, 0, 0, 0);
+            }
+        }
+        if (i >= STEPS) {  // four exponentials of P beside the dP products
+          const int e = i - STEPS, rb = e >> 3, kc = (e >> 2) & 1, th = (e >> 1) & 1, cb = e & 1;
+          const f32x4 l = *(const f32x4*)&st_s[0][wr * 64 + rb * 32 + kc * 16 + half * 8 + th * 4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const int at4 = kc * 8 + th * 4 + t;
+            st[rb][cb][at4] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[rb][cb][at4], c, -l[t]));
+          }
+        }
+        if (i + 1 < ALL) {
+          // the next step's copies are done; the last tile's stores were issued between the copies of steps 2 and 3
+          if (i + AHEAD >= ALL && !more) wait_vmcnt<0>();
+          else if (i < 2 && !start) wait_vmcnt<2 * COPIES + STORES>();
+          else wait_vmcnt<2 * COPIES>();
+          step_barrier();
+        }
+      }
+      const bool whole = k0 + kDsKeys <= s.lk && r0 >= s.first_row(p.right, k0 + kDsKeys - 1);
+#pragma unroll
+      for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int kc = 0; kc < 2; ++kc) {
+          const int lr = wr * 64 + rb * 32 + kc * 16 + half * 8;  // the chunk's first row in the tile
+          const f32x4 d0 = *(const f32x4*)&st_s[1][lr], d1 = *(const f32x4*)&st_s[1][lr + 4];
+#pragma unroll
+          for (int cb = 0; cb < 2; ++cb) {
+            float x[8], y[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+              x[t] = st[rb][cb][kc * 8 + t];
+              y[t] = x[t] * (dp[rb][cb][kc * 8 + t] + (t < 4 ? d0[t] : d1[t - 4]));
+            }
+            if (!whole) {
+              const int key = k0 + wc * 64 + cb * 32 + col;
+              const int first = key < s.lk ? s.first_row(p.right, key) : INT32_MAX;
+#pragma unroll
+              for (int t = 0; t < 8; ++t) {
+                const bool vis = r0 + lr + t >= first;
+                x[t] = vis ? x[t] : 0.f;
+                y[t] = vis ? y[t] : 0.f;
+              }
+            }
+            const uint32_t to = out_base + (uint32_t)cb * 2u * run + (uint32_t)(rb * 4 + kc * 2) * 256u + out_key[kc];
+            u32x4 px, dx;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              px[t] = pack_bf16(x[2 * t], x[2 * t + 1]);
+              dx[t] = pack_bf16(y[2 * t], y[2 * t + 1]);
+            }
+            __builtin_nontemporal_store(px, (u32x4*)(out_p + to));
+            __builtin_nontemporal_store(dx, (u32x4*)(out_s + to));
+          }
+        }
+      out_base += 8u * run;
+      ++kt;
+      if (!more) break;
+      k += k_tile;
+      v += v_tile;
+      keys = keys_next;
+      wait_vmcnt<2 * COPIES + STORES>();  // the copies of the next tile's first step
+      step_barrier();
+    }
+  }
+  if (kt < read) {  // the second half of a 256-key tile whose first half is seen: kernel 2 reads it
     const u32x4 zero = {0, 0, 0, 0};
 #pragma unroll
     for (int rb = 0; rb < 2; ++rb)
@@ -101,135 +262,18 @@ __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_ds_kernel(BwdWidePar
       for (int cb = 0; cb < 2; ++cb)
 #pragma unroll
         for (int kc = 0; kc < 2; ++kc) {
-          const uint32_t at = out_base + (uint32_t)cb * 2u * run + (uint32_t)(rb * 4 + kc * 2) * 256u + out_key[kc];
-          *(u32x4*)(out_p + at) = zero;
-          *(u32x4*)(out_s + at) = zero;
+          const uint32_t to = out_base + (uint32_t)cb * 2u * run + (uint32_t)(rb * 4 + kc * 2) * 256u + out_key[kc];
+          *(u32x4*)(out_p + to) = zero;
+          *(u32x4*)(out_s + to) = zero;
         }
-    return;
   }
-
-  {
-    const int row = r0 + (tid & 255), which = tid >> 8;
-    st_s[which][tid & 255] = row < s.lq ? p.stats[((int64_t)head * 2 + which) * p.total_q + s.qa + row]
-                                        : (which ? 0.f : INFINITY);  // a row past the sequence has P = 0
-  }
-  const int kvh = head / p.group;
-  const uint16_t* const q = p.q + (int64_t)(s.qa + r0) * p.sq_t + (int64_t)head * p.sq_h;
-  const uint16_t* const o = p.dout + (int64_t)(s.qa + r0) * p.sdo_t + (int64_t)head * p.sdo_h;
-  const uint16_t* const k = p.k + (int64_t)(s.ka + k0) * p.sk_t + (int64_t)kvh * p.sk_h;
-  const uint16_t* const v = p.v + (int64_t)(s.ka + k0) * p.sv_t + (int64_t)kvh * p.sv_h;
-  const int rows = min(s.lq - r0, kDsRows), keys = min(s.lk - k0, kDsKeys);
-  // tiles in the K layout of 64 columns: wave w copies A rows 32w .. +32 (four 1 KiB blocks: 16 rows x 64 B) and B
-  // rows 16w .. +16 (two)
-  const int lrow = lane & 15;
-  const uint32_t lcol = (uint32_t)(lane >> 4) * 16u;
-  const uint32_t q_off = (uint32_t)((wave * 32 + lrow) * (int)p.sq_t) * 2u + lcol;
-  const uint32_t o_off = (uint32_t)((wave * 32 + lrow) * (int)p.sdo_t) * 2u + lcol;
-  const uint32_t k_off = (uint32_t)((wave * 16 + lrow) * (int)p.sk_t) * 2u + lcol;
-  const uint32_t v_off = (uint32_t)((wave * 16 + lrow) * (int)p.sv_t) * 2u + lcol;
-  auto copy = [&](int step, KA_LDS char* a, KA_LDS char* b) {
-    const bool second = step >= STEPS;
-    const int at = (second ? step - STEPS : step) * kDsStep;
-    const uint16_t* const as = (second ? o : q) + at;
-    const uint16_t* const bs = (second ? v : k) + at;
-    const int a_t = (int)(second ? p.sdo_t : p.sq_t) * 2, b_t = (int)(second ? p.sv_t : p.sk_t) * 2;
-    const uint32_t a_off = second ? o_off : q_off, b_off = second ? v_off : k_off;
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      dma_16b(as, rows * a_t, a + (wave * 4 + r) * 1024, a_off + (uint32_t)((r >> 1) * 16 * a_t) + (r & 1) * 64u);
-#pragma unroll
-    for (int r = 0; r < 2; ++r) dma_16b(bs, keys * b_t, b + (wave * 2 + r) * 1024, b_off + r * 64u);
-  };
-  const int arow = key_row(col);
-  const int a_read = ((wr * 4 + (arow >> 4)) * 8 + half) * 256 + (arow & 15) * 16;  // + rb * 4096 + kk * 512
-  const int b_read = ((wc * 4 + (col >> 4)) * 8 + half) * 256 + (col & 15) * 16;    // + cb * 4096 + kk * 512
-
-  f32x16 st[2][2], dp[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      st[i][j] = f32x16{};
-      dp[i][j] = f32x16{};
-    }
-  auto products = [&](f32x16 (&acc)[2][2], const KA_LDS char* a, const KA_LDS char* b) {
-#pragma unroll
-    for (int kk = 0; kk < kDsStep / 16; ++kk) {
-      bf16x8 x[2], y[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        x[i] = *(const KA_LDS bf16x8*)(a + a_read + i * 4096 + kk * 512);
-        y[i] = *(const KA_LDS bf16x8*)(b + b_read + i * 4096 + kk * 512);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
-    }
-  };
-  KA_LDS char* const at[3] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s, (KA_LDS char*)a2_s};
-  KA_LDS char* const bt[3] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s, (KA_LDS char*)b2_s};
-  // a ring of three buffers: two steps of copies in flight
-  copy(0, at[0], bt[0]);
-  copy(1, at[1], bt[1]);
-  wait_vmcnt<6>();
-  step_barrier();
-#pragma unroll
-  for (int i = 0; i < 2 * STEPS; ++i) {
-    if (i + 2 < 2 * STEPS) copy(i + 2, at[(i + 2) % 3], bt[(i + 2) % 3]);
-    __builtin_amdgcn_sched_barrier(0);  // the copies are issued first
-    products(i < STEPS ? st : dp, at[i % 3], bt[i % 3]);
-    if (i + 1 < 2 * STEPS) {
-      if (i + 2 < 2 * STEPS) wait_vmcnt<6>(); else wait_vmcnt<0>();
-      step_barrier();
-    }
-  }
-
-  const float c = p.c;
-  const bool whole = k0 + kDsKeys <= s.lk && r0 >= s.first_row(p.right, k0 + kDsKeys - 1);
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc) {
-      const int lr = wr * 64 + rb * 32 + kc * 16 + half * 8;  // the chunk's first row in the tile
-      const f32x4 l0 = *(const f32x4*)&st_s[0][lr], l1 = *(const f32x4*)&st_s[0][lr + 4];
-      const f32x4 d0 = *(const f32x4*)&st_s[1][lr], d1 = *(const f32x4*)&st_s[1][lr + 4];
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        float x[8], y[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          x[t] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[rb][cb][kc * 8 + t], c, -(t < 4 ? l0[t] : l1[t - 4])));
-          y[t] = x[t] * (dp[rb][cb][kc * 8 + t] + (t < 4 ? d0[t] : d1[t - 4]));
-        }
-        if (!whole) {
-          const int key = k0 + wc * 64 + cb * 32 + col;
-          const int first = key < s.lk ? s.first_row(p.right, key) : INT32_MAX;
-#pragma unroll
-          for (int t = 0; t < 8; ++t) {
-            const bool vis = r0 + lr + t >= first;
-            x[t] = vis ? x[t] : 0.f;
-            y[t] = vis ? y[t] : 0.f;
-          }
-        }
-        const uint32_t to = out_base + (uint32_t)cb * 2u * run + (uint32_t)(rb * 4 + kc * 2) * 256u + out_key[kc];
-        u32x4 px, dx;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          px[t] = pack_bf16(x[2 * t], x[2 * t + 1]);
-          dx[t] = pack_bf16(y[2 * t], y[2 * t + 1]);
-        }
-        *(u32x4*)(out_p + to) = px;
-        *(u32x4*)(out_s + to) = dx;
-      }
-    }
 }
 
 // ---- kernel 2: a 256 x 256 output (256 columns of D, and 256 query rows of dQ or 256 keys of dK or dV) per
 // workgroup, eight waves of 128 (D) x 64
 template <bool DQ>
-__device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq& s, int item, KA_LDS char* const (&at)[2],
-                                          KA_LDS char* const (&bt)[2]) {
+__device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq& s, int item,
+                                          KA_LDS char* const (&at)[kRing], KA_LDS char* const (&bt)[kRing]) {
   const BwdParams& p = w.b;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -267,12 +311,11 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
     if (steps == 0 && !(last && !carry)) return;  // no row of the chunk sees these keys
   }
 
-  // copies: the A tile (64 keys or query rows x 256 columns of D, S layout): wave w copies columns (w & 1) * 128 ..
-  // of rows (w >> 1) * 16 .. +16; the B tile: dQ 64 keys x 256 rows, dK / dV 256 keys x 64 rows of P or dS
+  // copies: the A tile (32 keys or query rows x 256 columns of D, S layout): wave w copies columns (w & 3) * 64 .. of
+  // rows (w >> 2) * 16 .. +16; the B tile: dQ 32 keys x 256 rows, dK / dV 256 keys x 32 rows of P or dS
   const int64_t a_t = DQ ? p.sk_t : which ? p.sdo_t : p.sq_t;
   const int64_t a_h = which ? p.sdo_h : p.sq_h;
-  const uint32_t a_off = (uint32_t)(((wave >> 1) * 16 + ((lane & 15) ^ ((lane >> 4) << 2))) * (int)a_t) * 2u +
-                         (uint32_t)(wave & 1) * 256u + (uint32_t)(lane >> 4) * 16u;
+  const uint32_t a_off = s_block_base<kGradTile, 2>(wave, lane, a_t);
   const int64_t head_bytes = (int64_t)w.keys * w.rows * 2;
   const uint16_t* a_src;
   const char* b_src;
@@ -282,8 +325,8 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
     a_src = p.k + (int64_t)s.ka * a_t + (int64_t)(head / p.group) * p.sk_h + dhalf * 256;
     left_rows = s.lk;
     b_src = (const char*)w.ds + head * head_bytes + (int64_t)(n0 / 8) * 256;
-    b_off[0] = (uint32_t)(wave >> 1) * run + (uint32_t)(wave & 1) * 4096u + (uint32_t)lane * 16u;
-    b_off[1] = b_off[0] + 2048u;
+    b_off[0] = (uint32_t)(wave >> 2) * run + (uint32_t)(wave & 3) * 2048u + (uint32_t)lane * 16u;
+    b_off[1] = b_off[0] + 1024u;
   } else {
     a_src = (which ? p.dout : p.q) + (int64_t)(s.qa + first) * a_t + (int64_t)head * p.group * a_h + dhalf * 256;
     left_rows = s.lq - first;
@@ -300,9 +343,9 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
   auto copy = [&](KA_LDS char* a, KA_LDS char* b) {
     const int bytes = min(left_rows, kGradStep) * (int)a_t * 2;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      dma_16b(a_src, bytes, a + (wave * 4 + r) * 1024, a_off + r * 64u);
-      dma_16b((const uint16_t*)b_src, b_bytes, b + (wave * 4 + r) * 1024, b_off[r >> 1] + (r & 1) * 1024u);
+    for (int r = 0; r < 2; ++r) {
+      dma_16b(a_src, bytes, a + (wave * 2 + r) * 1024, s_block(a_off, r));
+      dma_16b((const uint16_t*)b_src, b_bytes, b + (wave * 2 + r) * 1024, b_off[r]);
     }
     a_src += a_step;
     b_src += b_step;
@@ -316,10 +359,11 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
       }
     }
   };
-  const int t_read[2] = {s_tr_base(lane, 0), s_tr_base(lane, 1)};  // + kc * 8192 + 32-column block * 1024
+  // transposed reads: + kc * 8192 + 32-column block * 1024
+  const int t_read[2] = {s_tr_base(lane, 0), s_tr_base(lane, 1)}, xt_read[2] = {x_tr_base(lane, 0), x_tr_base(lane, 1)};
   // dK / dV: chunk kc*2 + half of key wn*64 + j*32 + col
-  const int x_read[2] = {((wn * 4 + (col >> 4)) * 8 + half) * 256 + ((col & 15) ^ (half << 2)) * 16,
-                         ((wn * 4 + (col >> 4)) * 8 + 2 + half) * 256 + ((col & 15) ^ ((2 + half) << 2)) * 16};
+  const int x_read[2] = {((wn * 4 + (col >> 4)) * 4 + half) * 256 + ((col & 15) ^ (half << 2)) * 16,
+                         ((wn * 4 + (col >> 4)) * 4 + 2 + half) * 256 + ((col & 15) ^ ((2 + half) << 2)) * 16};
 
   f32x16 acc[4][2];
   f32x4* const kept = (f32x4*)w.acc + (int64_t)item * 32 * kWideThreads + tid;
@@ -339,45 +383,52 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
       }
     }
 
-  auto tr = [&](const KA_LDS char* t, int at) {
+  auto tr = [&](const KA_LDS char* t, const int (&base)[2], int at) {
     bf16x4 x[2];
 #pragma unroll
     for (int rr = 0; rr < 2; ++rr)
       x[rr] = __builtin_bit_cast(bf16x4,
-                                 __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(t + t_read[rr] + at)));
+                                 __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(t + base[rr] + at)));
     return __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7);
   };
   const int total = DQ ? steps : steps * p.group;
+  constexpr int AHEAD = kRing - 1, COPIES = 4;  // a wave's copies per step
   auto step = [&](int n, const KA_LDS char* a, const KA_LDS char* b, KA_LDS char* an, KA_LDS char* bn) {
-    if (n + 1 < total) copy(an, bn);
+    if (n + AHEAD < total) copy(an, bn);
     __builtin_amdgcn_sched_barrier(0);  // the copies are issued first
 #pragma unroll
     for (int kc = 0; kc < kGradStep / 16; ++kc) {
       bf16x8 x[4], y[2];
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        if constexpr (DQ) y[j] = tr(b, kc * 8192 + wn * 2048 + j * 1024);
-        else y[j] = *(const KA_LDS bf16x8*)(b + x_read[kc & 1] + (kc >> 1) * 1024 + j * 4096);
+        if constexpr (DQ) y[j] = tr(b, xt_read, kc * 8192 + wn * 2048 + j * 1024);
+        else y[j] = *(const KA_LDS bf16x8*)(b + x_read[kc] + j * 2048);
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = tr(a, kc * 8192 + wd * 4096 + i * 1024);
+      for (int i = 0; i < 4; ++i) x[i] = tr(a, t_read, kc * 8192 + wd * 4096 + i * 1024);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
     }
-    wait_vmcnt<0>();
+    // the next step's copies are done (those of up to two later steps may be in flight)
+    if (n + AHEAD < total) wait_vmcnt<2 * COPIES>();
+    else if (n + 2 < total) wait_vmcnt<COPIES>();
+    else wait_vmcnt<0>();
     step_barrier();
   };
-  if (total > 0) copy(at[0], bt[0]);
-  wait_vmcnt<0>();
-  __syncthreads();
-  int n = 0;
-  for (; n + 1 < total; n += 2) {
-    step(n, at[0], bt[0], at[1], bt[1]);
-    step(n + 1, at[1], bt[1], at[0], bt[0]);
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+    if (i < total) copy(at[i], bt[i]);
+  if (total > 2) wait_vmcnt<2 * COPIES>();
+  else wait_vmcnt<0>();
+  step_barrier();
+  for (int n = 0; n < total; n += kRing) {
+    step(n, at[0], bt[0], at[3], bt[3]);
+    if (n + 1 < total) step(n + 1, at[1], bt[1], at[0], bt[0]);
+    if (n + 2 < total) step(n + 2, at[2], bt[2], at[1], bt[1]);
+    if (n + 3 < total) step(n + 3, at[3], bt[3], at[2], bt[2]);
   }
-  if (n < total) step(n, at[0], bt[0], at[1], bt[1]);
 
   if (!DQ && !last) {
 #pragma unroll
@@ -416,9 +467,10 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
 
 __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_grad_kernel(BwdWideParams w) {
   constexpr int TILE = kGradStep * kGradTile * 2;
-  __shared__ __attribute__((aligned(1024))) char a0_s[TILE], a1_s[TILE], b0_s[TILE], b1_s[TILE];
-  KA_LDS char* const at[2] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s};
-  KA_LDS char* const bt[2] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s};
+  __shared__ __attribute__((aligned(1024))) char a0_s[TILE], a1_s[TILE], a2_s[TILE], a3_s[TILE];
+  __shared__ __attribute__((aligned(1024))) char b0_s[TILE], b1_s[TILE], b2_s[TILE], b3_s[TILE];
+  KA_LDS char* const at[kRing] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s, (KA_LDS char*)a2_s, (KA_LDS char*)a3_s};
+  KA_LDS char* const bt[kRing] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s, (KA_LDS char*)b2_s, (KA_LDS char*)b3_s};
   const WideSeq s(w);
   const int dq_items = w.rows / kGradTile * 2 * w.b.heads;
   if ((int)blockIdx.x < dq_items) wide_grad<true>(w, s, blockIdx.x, at, bt);
@@ -427,7 +479,11 @@ __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_grad_kernel(BwdWideP
 
 hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream) {
   const int kv_heads = w.b.heads / w.b.group;
-  const int64_t ds_items = (int64_t)(w.rows / kDsRows) * (w.keys / kDsKeys) * w.b.heads;
+  // key tiles per workgroup of kernel 1: at least 1,024 workgroups (four per CU), at most eight tiles
+  const int64_t row_tiles = (int64_t)(w.rows / kDsRows) * w.b.heads, key_tiles = w.keys / kDsKeys;
+  const int64_t per = row_tiles * key_tiles / 1024;
+  w.run = (int32_t)(per < 1 ? 1 : per > 8 ? 8 : per);
+  const int64_t ds_items = row_tiles * ((key_tiles + w.run - 1) / w.run);
   const int64_t grad_items = (int64_t)(w.rows / kGradTile) * 2 * w.b.heads + (int64_t)(w.keys / kGradTile) * 4 * kv_heads;
   for (int64_t r = 0; r < w.b.total_q; r += w.rows) {
     w.r_begin = (int32_t)r;

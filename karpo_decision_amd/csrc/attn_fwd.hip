@@ -483,7 +483,9 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
   };
 
   // ---- LDS read bases (per lane) for the MFMA operands (a pair's second wave starts at the second half of D)
-  const int k_read = k_offset<D>(key_row(col), half) + dh * QC * 512;  // + kb * (2 * D/8 * 256) + dc * 512
+  // K: k_read[dc & 1] + kb * (2 * D/8 * 256) + (dc >> 1) * 1024
+  const int k_read[2] = {s_offset<D>(key_row(col), half) + dh * QC * 512,
+                         s_offset<D>(key_row(col), 2 + half) + dh * QC * 512};
   const int g = lane >> 4, jl = lane & 15;
   const int v_read =
       v_offset<D>(8 * (g >> 1) + (jl >> 2), 16 * (g & 1) + 4 * (jl & 3)) + dh * OB * 256;  // + kc, rr, db offsets
@@ -568,7 +570,7 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
       for (int dc = 0; dc < QC; ++dc) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
-          const bf16x8 a = *(const KA_LDS bf16x8*)(kt + k_read + kb * (2 * (D / 8) * 256) + dc * 512);
+          const bf16x8 a = *(const KA_LDS bf16x8*)(kt + k_read[dc & 1] + kb * (2 * (D / 8) * 256) + (dc >> 1) * 1024);
 #pragma unroll
           for (int b = 0; b < QB; ++b)  // one K operand read feeds every query block
             st[b][kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qop[b][dc], st[b][kb], 0, 0, 0);
@@ -926,7 +928,8 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_pair_pp_kernel(Params p) {
     jt += BN;
   };
 
-  const int k_read = k_offset<D>(key_row(col), half) + dh * QC * 512;
+  const int k_read[2] = {s_offset<D>(key_row(col), half) + dh * QC * 512,
+                         s_offset<D>(key_row(col), 2 + half) + dh * QC * 512};
   const int g = lane >> 4, jl = lane & 15;
   const int v_read = v_offset<D>(8 * (g >> 1) + (jl >> 2), 16 * (g & 1) + 4 * (jl & 3)) + dh * OB * 256;
 
@@ -954,7 +957,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_pair_pp_kernel(Params p) {
       st = f32x16{};
 #pragma unroll
       for (int dc = 0; dc < QC; ++dc) {
-        const bf16x8 a = *(const KA_LDS bf16x8*)(kt + k_read + dc * 512);
+        const bf16x8 a = *(const KA_LDS bf16x8*)(kt + k_read[dc & 1] + (dc >> 1) * 1024);
         st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qop[dc], st, 0, 0, 0);
       }
     }

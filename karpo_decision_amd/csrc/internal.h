@@ -89,6 +89,7 @@ struct BwdWideParams {
   int32_t rows;     // query rows per chunk, a multiple of 256
   int32_t keys;     // total_k rounded up to 256
   int32_t r_begin;  // the chunk's first query row (set by the launch)
+  int32_t run;      // key tiles per workgroup of the first kernel (set by the launch)
 };
 hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream);
 // items_q / items_k: the work lists' item capacities (the grids), tiles_q / tiles_k their tile capacities, merges_k

@@ -28,11 +28,8 @@ constexpr int kBufferFlags = 0x00020000;
 // Row of the 32-key block that MFMA A-row r reads: bits 2 and 3 of r swapped.
 __device__ __forceinline__ int key_row(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
 
-// Byte offsets inside the LDS tiles.
-//   K: (key k, 16-byte chunk c of its D/8) at ((k / 16) * D/8 + c) * 256 + (k % 16) * 16
-//   V: (key k, element d) at ((k / 4) * D/16 + d / 16) * 128 + (k % 4) * 32 + (d % 16) * 2
-template <int D>
-__device__ __forceinline__ int k_offset(int k, int c) { return ((k >> 4) * (D / 8) + c) * 256 + (k & 15) * 16; }
+// Byte offset inside the forward's V tile: (key k, element d) at
+// ((k / 4) * D/16 + d / 16) * 128 + (k % 4) * 32 + (d % 16) * 2. Its K tile is in the S layout (s_offset).
 template <int D>
 __device__ __forceinline__ int v_offset(int k, int d) {
   return ((k >> 2) * (D / 16) + (d >> 4)) * 128 + (k & 3) * 32 + (d & 15) * 2;
@@ -63,30 +60,40 @@ __device__ __forceinline__ int wave_max(int x) {
 }
 
 // The S layout: rows (keys, or query rows) staged once and read both as MFMA row operands (ds_read_b128, one row's
-// 16-byte chunk per lane) and transposed (ds_read_b64_tr_b16, four rows of one column group per lane). Chunk c of
-// row k sits at ((k / 16) * D/8 + c) * 256 + ((k % 16) ^ 4 (c % 4)) * 16: a 256 B run holds 16 rows' chunk c, with the
-// rows' order XOR-swizzled by the chunk index, so the 16 lanes of a row read cover one run and the 32 lanes of a
-// transposed read (four rows x chunks c .. c+3) cover 64 distinct banks.
+// 16-byte chunk per lane) and transposed (ds_read_b64_tr_b16, four rows of one column group per lane). 16 rows x 4
+// chunks (64 B) make a 1 KiB block; in it row k's 64 B sit at (k % 16) * 64, its chunks XOR-swizzled by k / 4:
+//   s_offset = ((k / 16) * D/32 + c / 4) * 1024 + (k % 16) * 64 + ((c % 4) ^ (k / 4 % 4)) * 16.
+// The 16 lanes of a row read (16 rows, one chunk) cover 64 distinct banks, and the 32 lanes of a transposed read (four
+// rows x chunks c .. c+3) one contiguous 256 B run. Four consecutive lanes of a copy read 64 consecutive bytes: a
+// copy instruction whose neighbouring lanes read different rows takes the address unit a cycle per lane whatever its
+// total (9.5 TB/s out of L2 over the GPU, against 20-31 for 64 B and 31 for 128 B per row; 1 MiB read by 256
+// workgroups), which bounded the kernels while chunk c of 16 rows made a 256 B run.
 template <int D>
-__device__ __forceinline__ int s_offset(int k, int c) {
-  return ((k >> 4) * (D / 8) + c) * 256 + (((k & 15) ^ ((c & 3) << 2)) * 16);
+KA_HD inline int s_offset(int k, int c) {
+  return ((k >> 4) * (D / 32) + (c >> 2)) * 1024 + (k & 15) * 64 + ((c & 3) ^ ((k >> 2) & 3)) * 16;
 }
 // Inverse of s_offset for byte offset blk * 1024 + lane * 16 (the copy's source row and first column).
 template <int D>
-__device__ __forceinline__ void s_dma_source(int blk, int lane, int* row, int* col) {
-  const int b = blk * 4 + (lane >> 4);  // 256-byte run: (row block, chunk)
-  const int c = b % (D / 8);
-  *row = (b / (D / 8)) * 16 + ((lane & 15) ^ ((c & 3) << 2));
-  *col = c * 8;
+KA_HD inline void s_dma_source(int blk, int lane, int* row, int* col) { k_dma_source<D>(blk, lane, row, col); }
+// A wave's INSTS consecutive blocks (blocks INSTS * wave ..) lie in the same 16 rows, 64 B apart: the byte offset of
+// its first, from the tile's first row, serves them all (one register per tile).
+template <int D, int INSTS>
+KA_HD inline uint32_t s_block_base(int wave, int lane, int64_t stride) {
+  static_assert((D / 32) % INSTS == 0, "the wave's blocks lie in one block of 16 rows");
+  int row, col;
+  s_dma_source<D>(wave * INSTS, lane, &row, &col);
+  return (uint32_t)(row * stride + col) * 2u;
 }
+KA_HD inline uint32_t s_block(uint32_t base, int r) { return base + (uint32_t)r * 64u; }
 // Row-operand read of element chunk 2 dc + half of row k: s_offset(k, 2 dc + half) = base[dc & 1] + (dc >> 1) * 1024
 // with base[i] = s_offset(k, 2 i + half).
 // Transposed read (the A operand rows d = db*32 + lane%32 over rows kc*16 + (lane/32)*8 .. +8 of the step, two reads
 // rr = 0, 1 of four rows each): this lane's address is s_tr_base(lane, rr) + kc * (D/8) * 256 + db * 1024.
-__device__ __forceinline__ int s_tr_base(int lane, int rr) {
+KA_HD inline int s_tr_base(int lane, int rr) {
   const int g = lane >> 4, jl = lane & 15;
-  const int c = 2 * (g & 1) + ((jl >> 1) & 1);  // chunk within the 32-column block (its index mod 4)
-  return c * 256 + (((4 * rr + 8 * (g >> 1) + (jl >> 2)) ^ (c << 2)) * 16) + (jl & 1) * 8;
+  const int c = 2 * (g & 1) + ((jl >> 1) & 1);           // chunk within the 32-column block
+  const int row = 4 * rr + 8 * (g >> 1) + (jl >> 2);
+  return row * 64 + (c ^ (row >> 2)) * 16 + (jl & 1) * 8;
 }
 
 // s_waitcnt vmcnt(N) (expcnt and lgkmcnt not waited on): at most N vector-memory operations of this wave in flight.

@@ -10,15 +10,15 @@
 
 namespace karpo {
 
-// Where lane `lane` of DMA instruction `blk` (1 KiB of the K tile each) reads: the key row inside the step and the
-// element column. The inverse of k_offset (mfma_common.h) for byte offset blk * 1024 + lane * 16.
+// Where lane `lane` of DMA instruction `blk` (1 KiB of the K tile each: 16 keys x 64 B) reads: the key row inside the
+// step and the element column. The inverse of s_offset (mfma_common.h) for byte offset blk * 1024 + lane * 16: four
+// consecutive lanes read 64 consecutive bytes of one key.
 template <int D>
 KA_HD inline void k_dma_source(int blk, int lane, int* key, int* col) {
-  const int b = blk * 4 + (lane >> 4);  // 256-byte block: (key block, chunk)
-  *key = (b / (D / 8)) * 16 + (lane & 15);
-  *col = (b % (D / 8)) * 8;
+  *key = (blk / (D / 32)) * 16 + (lane >> 2);
+  *col = (blk % (D / 32)) * 32 + ((lane & 3) ^ (lane >> 4)) * 8;
 }
-// The same for the V tile (the inverse of v_offset).
+// The same for the V tile (the inverse of v_offset): two consecutive lanes read 32 consecutive bytes.
 template <int D>
 KA_HD inline void v_dma_source(int blk, int lane, int* key, int* col) {
   const int b = blk * 8 + (lane >> 3);  // 128-byte block: (key group, d block)

@@ -497,9 +497,13 @@ def packed_attention_backward(grad: Tensor, query: Tensor, key: Tensor, value: T
         b.d_q, b.d_q_stride_tok, b.d_q_stride_head = dq.data_ptr(), dq.stride(0), dq.stride(1)
         b.d_k, b.d_k_stride_tok, b.d_k_stride_head = dk.data_ptr(), dk.stride(0), dk.stride(1)
         b.d_v, b.d_v_stride_tok, b.d_v_stride_head = dv.data_ptr(), dv.stride(0), dv.stride(1)
-        try:  # the workspace of the fastest path where the device has it, else the least the call runs in
-            workspace = _workspace(lib, lib.karpo_attn_bwd_workspace_best_bytes, b, query.device)
-        except torch.OutOfMemoryError:
+        workspace = None
+        if query.shape[2] == 512:  # the workspace of the fastest path where the device has it
+            try:
+                workspace = _workspace(lib, lib.karpo_attn_bwd_workspace_best_bytes, b, query.device)
+            except torch.OutOfMemoryError:
+                pass
+        if workspace is None:
             workspace = _workspace(lib, lib.karpo_attn_bwd_workspace_bytes, b, query.device)
         b.fwd.workspace, b.fwd.workspace_bytes = workspace.data_ptr(), workspace.numel()
         stream = _current_stream(query.device.index)
