@@ -9,7 +9,7 @@
 // 5,120 FLOPs need them, so keeping them takes less time than either the recomputation or the exchange: five products,
 // each a plain tiled matrix product with every accumulator in one wave's registers. Measured against the wave pairs
 // (32 / 4 heads, causal, MI355X): 497 -> 140 us at 512 rows, 2.09 -> 0.83 ms at 2,048, 12.4 -> 8.0 ms at 8,192, 48.1 ->
-// 26.2 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
+// 24.4 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
 // call takes this path when the workspace has room for a chunk of 256 rows.
 //
 // P and dS in the workspace: per head [key block of 16][chunk of 8 rows][16 keys][8 rows] bf16, the 16 keys of a
@@ -25,6 +25,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "bwd_common.h"
 #include "internal.h"
 #include "karpo_attn.h"
@@ -34,7 +36,8 @@
 namespace karpo {
 
 constexpr int kWideD = 512;
-constexpr int kWideThreads = 512;               // eight waves
+constexpr int kWideThreads = 512;               // kernel 1: eight waves
+constexpr int kGradThreads = 256;               // kernel 2: four waves
 constexpr int kDsRows = 256, kDsKeys = 128;     // kernel 1's tile
 constexpr int kDsStep = 32;                     // elements of D per step
 constexpr int kGradTile = 256, kGradStep = 32;  // kernel 2's outputs (both ways) and contraction step
@@ -269,17 +272,24 @@ __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_ds_kernel(BwdWidePar
   }
 }
 
-// ---- kernel 2: a 256 x 256 output (256 columns of D, and 256 query rows of dQ or 256 keys of dK or dV) per
-// workgroup, eight waves of 128 (D) x 64
+// ---- kernel 2: a 256 x 256 output (256 columns of D, and 256 query rows of dQ or 256 keys of dK or dV) per workgroup,
+// four waves of 128 x 128 (one per SIMD, 256 accumulators in AGPRs): each operand read from LDS feeds four MFMAs. The
+// operands of a half step (16 of the contraction) are read during the MFMAs of the half step before it; the barrier
+// that publishes a step's copies is passed halfway through the step before, when every wave has read the whole of
+// that step's buffer, so the copies of three to four steps are in flight. The chunk of the last 2,048 of 16,384 rows
+// (32 / 4 heads): 3.13 ms with eight waves of 128 x 64, 2.88 ms so, 2.50 ms with the reads and copies spread between the
+// MFMAs (sched_group_barrier); 1.4 ms at the nominal MFMA rate.
 template <bool DQ>
 __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq& s, int item,
                                           KA_LDS char* const (&at)[kRing], KA_LDS char* const (&bt)[kRing]) {
+  constexpr int W = kGradThreads / 64, INSTS = kGradStep * kGradTile * 2 / 1024 / W;
+  constexpr int COPIES = 2 * INSTS;  // a wave's copies per step
   const BwdParams& p = w.b;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 31, half = lane >> 5;
-  const int wd = wave >> 2, wn = wave & 3;
-  const uint32_t run = (uint32_t)(w.rows / 8) * 256u;
+  const int wd = wave >> 1, wn = wave & 1;
+  const int64_t run = (int64_t)(w.rows / 8) * 256;  // bytes per block of 16 keys of P or dS
   const int r_end = min(s.lq, w.r_begin + w.rows);
 
   int head, dhalf, n0, which = 0, steps, first = 0;  // n0: the first query row (dQ, from the chunk's first) or key
@@ -311,77 +321,68 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
     if (steps == 0 && !(last && !carry)) return;  // no row of the chunk sees these keys
   }
 
-  // copies: the A tile (32 keys or query rows x 256 columns of D, S layout): wave w copies columns (w & 3) * 64 .. of
-  // rows (w >> 2) * 16 .. +16; the B tile: dQ 32 keys x 256 rows, dK / dV 256 keys x 32 rows of P or dS
+  // copies: the A tile (32 keys or query rows x 256 columns of D, S layout): wave w copies columns (w & 1) * 128 .. of
+  // rows (w >> 1) * 16 .. +16; the B tile: dQ 32 keys x 256 rows, dK / dV 256 keys x 32 rows of P or dS
   const int64_t a_t = DQ ? p.sk_t : which ? p.sdo_t : p.sq_t;
   const int64_t a_h = which ? p.sdo_h : p.sq_h;
-  const uint32_t a_off = s_block_base<kGradTile, 2>(wave, lane, a_t);
+  const uint32_t a_off = s_block_base<kGradTile, INSTS>(wave, lane, a_t), b_off = (uint32_t)lane * 16u;
   const int64_t head_bytes = (int64_t)w.keys * w.rows * 2;
   const uint16_t* a_src;
   const char* b_src;
   int left_rows, in_head = 0;
-  uint32_t b_off[2];
   if constexpr (DQ) {
     a_src = p.k + (int64_t)s.ka * a_t + (int64_t)(head / p.group) * p.sk_h + dhalf * 256;
     left_rows = s.lk;
-    b_src = (const char*)w.ds + head * head_bytes + (int64_t)(n0 / 8) * 256;
-    b_off[0] = (uint32_t)(wave >> 2) * run + (uint32_t)(wave & 3) * 2048u + (uint32_t)lane * 16u;
-    b_off[1] = b_off[0] + 1024u;
+    b_src = (const char*)w.ds + head * head_bytes + (int64_t)(n0 / 8) * 256 + (wave >> 1) * run + (wave & 1) * 4096;
   } else {
     a_src = (which ? p.dout : p.q) + (int64_t)(s.qa + first) * a_t + (int64_t)head * p.group * a_h + dhalf * 256;
     left_rows = s.lq - first;
-    b_src = (const char*)(which ? w.p : w.ds) + (int64_t)head * p.group * head_bytes + (int64_t)(n0 / 16) * run +
-            (int64_t)((first - w.r_begin) / 8) * 256;
-    b_off[0] = (uint32_t)(wave * 2) * run + (uint32_t)lane * 16u;
-    b_off[1] = b_off[0] + run;
+    b_src = (const char*)(which ? w.p : w.ds) + (int64_t)head * p.group * head_bytes +
+            (int64_t)(n0 / 16 + wave * INSTS) * run + (int64_t)((first - w.r_begin) / 8) * 256;
   }
   const int64_t a_step = (int64_t)kGradStep * a_t;
-  const int64_t b_step = DQ ? (int64_t)(kGradStep / 16) * run : (int64_t)(kGradStep / 8) * 256;
-  const int b_bytes = (int)((DQ ? kGradStep / 16 : kGradTile / 16) * run);
-  const int64_t a_wrap = a_h - steps * a_step, b_wrap = head_bytes - steps * b_step;
+  const int64_t b_step = DQ ? (kGradStep / 16) * run : (int64_t)(kGradStep / 8) * 256;
+  const int64_t b_block = DQ ? 1024 : run;
+  const int64_t a_wrap = a_h - (steps - 1) * a_step, b_wrap = head_bytes - (steps - 1) * b_step;
   const int top_rows = left_rows;
   auto copy = [&](KA_LDS char* a, KA_LDS char* b) {
     const int bytes = min(left_rows, kGradStep) * (int)a_t * 2;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      dma_16b(a_src, bytes, a + (wave * 2 + r) * 1024, s_block(a_off, r));
-      dma_16b((const uint16_t*)b_src, b_bytes, b + (wave * 2 + r) * 1024, b_off[r]);
+    for (int r = 0; r < INSTS; ++r) {
+      dma_16b(a_src, bytes, a + (wave * INSTS + r) * 1024, s_block(a_off, r));
+      dma_16b((const uint16_t*)(b_src + r * b_block), 1024, b + (wave * INSTS + r) * 1024, b_off);
     }
-    a_src += a_step;
-    b_src += b_step;
-    left_rows -= kGradStep;
-    if constexpr (!DQ) {
-      if (++in_head == steps) {  // the group's next head
-        in_head = 0;
-        a_src += a_wrap;
-        b_src += b_wrap;
-        left_rows = top_rows;
-      }
-    }
+    const bool wrap = !DQ && in_head + 1 == steps;  // the group's next head
+    in_head = wrap ? 0 : in_head + 1;
+    a_src += wrap ? a_wrap : a_step;
+    b_src += wrap ? b_wrap : b_step;
+    left_rows = wrap ? top_rows : left_rows - kGradStep;
   };
   // transposed reads: + kc * 8192 + 32-column block * 1024
-  const int t_read[2] = {s_tr_base(lane, 0), s_tr_base(lane, 1)}, xt_read[2] = {x_tr_base(lane, 0), x_tr_base(lane, 1)};
-  // dK / dV: chunk kc*2 + half of key wn*64 + j*32 + col
-  const int x_read[2] = {((wn * 4 + (col >> 4)) * 4 + half) * 256 + ((col & 15) ^ (half << 2)) * 16,
-                         ((wn * 4 + (col >> 4)) * 4 + 2 + half) * 256 + ((col & 15) ^ ((2 + half) << 2)) * 16};
+  const int t_read[2] = {s_tr_base(lane, 0) + wd * 4096, s_tr_base(lane, 1) + wd * 4096};
+  const int xt_read[2] = {x_tr_base(lane, 0) + wn * 4096, x_tr_base(lane, 1) + wn * 4096};
+  // dK / dV: chunk kc*2 + half of key wn*128 + j*32 + col
+  const int x_read[2] = {((wn * 8 + (col >> 4)) * 4 + half) * 256 + ((col & 15) ^ (half << 2)) * 16,
+                         ((wn * 8 + (col >> 4)) * 4 + 2 + half) * 256 + ((col & 15) ^ ((2 + half) << 2)) * 16};
 
-  f32x16 acc[4][2];
-  f32x4* const kept = (f32x4*)w.acc + (int64_t)item * 32 * kWideThreads + tid;
-  const bool any = !DQ && carry;
+  f32x16 acc[4][4];
+  f32x4* const kept = (f32x4*)w.acc + (int64_t)item * 64 * kGradThreads + tid;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      acc[i][j] = f32x16{};
-      if (any) {
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x16{};
+  if (!DQ && carry) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const f32x4 x = kept[((i * 2 + j) * 4 + g) * kWideThreads];
+          const f32x4 x = kept[((i * 4 + j) * 4 + g) * kGradThreads];
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[i][j][g * 4 + e] = x[e];
         }
-      }
-    }
+  }
 
   auto tr = [&](const KA_LDS char* t, const int (&base)[2], int at) {
     bf16x4 x[2];
@@ -391,61 +392,94 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
                                  __builtin_amdgcn_ds_read_tr16_b64_v4i16((KA_LDS s16x4*)(t + base[rr] + at)));
     return __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7);
   };
-  const int total = DQ ? steps : steps * p.group;
-  constexpr int AHEAD = kRing - 1, COPIES = 4;  // a wave's copies per step
-  auto step = [&](int n, const KA_LDS char* a, const KA_LDS char* b, KA_LDS char* an, KA_LDS char* bn) {
-    if (n + AHEAD < total) copy(an, bn);
-    __builtin_amdgcn_sched_barrier(0);  // the copies are issued first
+  bf16x8 x[2][4], y[2][4];  // the operands of the two half steps
+  auto read = [&](int kc, const KA_LDS char* a, const KA_LDS char* b) {
 #pragma unroll
-    for (int kc = 0; kc < kGradStep / 16; ++kc) {
-      bf16x8 x[4], y[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if constexpr (DQ) y[j] = tr(b, xt_read, kc * 8192 + wn * 2048 + j * 1024);
-        else y[j] = *(const KA_LDS bf16x8*)(b + x_read[kc] + j * 2048);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[i] = tr(a, t_read, kc * 8192 + wd * 4096 + i * 1024);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[i], y[j], acc[i][j], 0, 0, 0);
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (DQ) y[kc][i] = tr(b, xt_read, kc * 8192 + i * 1024);
+      else y[kc][i] = *(const KA_LDS bf16x8*)(b + x_read[kc] + i * 2048);
+      x[kc][i] = tr(a, t_read, kc * 8192 + i * 1024);
     }
-    // the next step's copies are done (those of up to two later steps may be in flight)
-    if (n + AHEAD < total) wait_vmcnt<2 * COPIES>();
+  };
+  auto multiply = [&](int kc) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[kc][i], y[kc][j], acc[i][j], 0, 0, 0);
+  };
+  const int total = DQ ? steps : steps * p.group;
+  // step n in buffer a, b (an, bn: step n + 1's); its first half's operands are read
+  // (FULL: so are steps n + 1 to n + 4 there)
+  auto step = [&](auto full, int n, KA_LDS char* a, KA_LDS char* b, const KA_LDS char* an, const KA_LDS char* bn) {
+    constexpr bool FULL = decltype(full)::value;
+    read(1, a, b);
+    multiply(0);
+    if constexpr (FULL) {  // LDS reads (0x100) and copies (0x020) issued between the MFMAs (0x008)
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (FULL || n + 3 < total) wait_vmcnt<2 * COPIES>();  // step n + 1's copies; two later steps' may be in flight
     else if (n + 2 < total) wait_vmcnt<COPIES>();
     else wait_vmcnt<0>();
     step_barrier();
+    if (FULL || n + kRing < total) copy(a, b);
+    if (FULL || n + 1 < total) read(0, an, bn);
+    multiply(1);
+    if constexpr (FULL) {
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
-  for (int i = 0; i < AHEAD; ++i)
+  for (int i = 0; i < kRing; ++i)
     if (i < total) copy(at[i], bt[i]);
-  if (total > 2) wait_vmcnt<2 * COPIES>();
+  if (total > 3) wait_vmcnt<3 * COPIES>();
   else wait_vmcnt<0>();
   step_barrier();
-  for (int n = 0; n < total; n += kRing) {
-    step(n, at[0], bt[0], at[3], bt[3]);
-    if (n + 1 < total) step(n + 1, at[1], bt[1], at[0], bt[0]);
-    if (n + 2 < total) step(n + 2, at[2], bt[2], at[1], bt[1]);
-    if (n + 3 < total) step(n + 3, at[3], bt[3], at[2], bt[2]);
+  if (total > 0) read(0, at[0], bt[0]);
+  int n = 0;
+  const std::true_type full;
+  const std::false_type tail;
+  for (; n + 2 * kRing <= total; n += kRing) {
+    step(full, n, at[0], bt[0], at[1], bt[1]);
+    step(full, n + 1, at[1], bt[1], at[2], bt[2]);
+    step(full, n + 2, at[2], bt[2], at[3], bt[3]);
+    step(full, n + 3, at[3], bt[3], at[0], bt[0]);
+  }
+  for (; n < total; n += kRing) {
+    step(tail, n, at[0], bt[0], at[1], bt[1]);
+    if (n + 1 < total) step(tail, n + 1, at[1], bt[1], at[2], bt[2]);
+    if (n + 2 < total) step(tail, n + 2, at[2], bt[2], at[3], bt[3]);
+    if (n + 3 < total) step(tail, n + 3, at[3], bt[3], at[0], bt[0]);
   }
 
   if (!DQ && !last) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          kept[((i * 2 + j) * 4 + g) * kWideThreads] =
+          kept[((i * 4 + j) * 4 + g) * kGradThreads] =
               f32x4{acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
     return;
   }
-  // lane (col, half) holds d = dhalf*256 + wd*128 + i*32 + (reg/4)*8 + half*4 + reg%4 of row / key wn*64 + j*32 + col
+  // lane (col, half) holds d = dhalf*256 + wd*128 + i*32 + (reg/4)*8 + half*4 + reg%4 of row / key wn*128 + j*32 + col
   const float scale = DQ || which == 0 ? p.scale : 1.f;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int at_n = n0 + wn * 64 + j * 32 + col;
+  for (int j = 0; j < 4; ++j) {
+    const int at_n = n0 + wn * 128 + j * 32 + col;
     const bool valid = DQ ? w.r_begin + at_n < s.lq : at_n < s.lk;
     uint16_t* to;
     if constexpr (DQ) to = p.dq + (int64_t)(s.qa + w.r_begin + at_n) * p.sdq_t + (int64_t)head * p.sdq_h;
@@ -457,15 +491,15 @@ __device__ __forceinline__ void wide_grad(const BwdWideParams& w, const WideSeq&
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        u32x2 x;
-        x[0] = pack_bf16(acc[i][j][g * 4] * scale, acc[i][j][g * 4 + 1] * scale);
-        x[1] = pack_bf16(acc[i][j][g * 4 + 2] * scale, acc[i][j][g * 4 + 3] * scale);
-        *(u32x2*)(to + i * 32 + g * 8) = x;
+        u32x2 o;
+        o[0] = pack_bf16(acc[i][j][g * 4] * scale, acc[i][j][g * 4 + 1] * scale);
+        o[1] = pack_bf16(acc[i][j][g * 4 + 2] * scale, acc[i][j][g * 4 + 3] * scale);
+        *(u32x2*)(to + i * 32 + g * 8) = o;
       }
   }
 }
 
-__global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_grad_kernel(BwdWideParams w) {
+__global__ __launch_bounds__(kGradThreads, 1) void bwd_wide_grad_kernel(BwdWideParams w) {
   constexpr int TILE = kGradStep * kGradTile * 2;
   __shared__ __attribute__((aligned(1024))) char a0_s[TILE], a1_s[TILE], a2_s[TILE], a3_s[TILE];
   __shared__ __attribute__((aligned(1024))) char b0_s[TILE], b1_s[TILE], b2_s[TILE], b3_s[TILE];
@@ -490,7 +524,7 @@ hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream) {
     hipLaunchKernelGGL(bwd_wide_ds_kernel, dim3((unsigned)ds_items), dim3(kWideThreads), 0, stream, w);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bwd_wide_grad_kernel, dim3((unsigned)grad_items), dim3(kWideThreads), 0, stream, w);
+    hipLaunchKernelGGL(bwd_wide_grad_kernel, dim3((unsigned)grad_items), dim3(kGradThreads), 0, stream, w);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
