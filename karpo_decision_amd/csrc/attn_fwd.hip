@@ -1173,50 +1173,55 @@ __global__ __launch_bounds__(kMergeThreads) void merge_kernel(Params p) {
 // ---- device planner: one workgroup turns the device bounds into the longest-first work list.
 
 constexpr int kPlanThreads = 1024;
+constexpr int kPlanSeqs = 1024;  // sequences whose bounds the planner holds in LDS
 
-__device__ int block_exclusive_scan(int x, int* total, int* scratch /* >= kPlanThreads/64 + 1 */) {
+constexpr int kPlanWaves = kPlanThreads / 64;
+
+// The sum over the block of x before this thread's, and in *total the whole sum. One barrier: every thread adds up the
+// waves' sums itself (independent broadcast reads; a serial loop in one thread between two barriers took 0.7 us). Calls
+// in a row take different `scratch`.
+template <class T>
+__device__ __forceinline__ T block_exclusive_scan(T x, T* total, T* scratch /* kPlanWaves */) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int incl = x;
+  T incl = x;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(incl, o);
+    const T y = __shfl_up(incl, o);
     if (lane >= o) incl += y;
   }
   if (lane == 63) scratch[wave] = incl;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int w = 0; w < kPlanThreads / 64; ++w) {
-      const int t = scratch[w];
-      scratch[w] = run;
-      run += t;
-    }
-    scratch[kPlanThreads / 64] = run;
+  T before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < kPlanWaves; ++w) {
+    const T t = scratch[w];
+    before += w < wave ? t : 0;
+    all += t;
   }
-  __syncthreads();
-  const int ex = scratch[wave] + incl - x;
-  *total = scratch[kPlanThreads / 64];
-  __syncthreads();
-  return ex;
+  *total = all;
+  return before + incl - x;
 }
 
-__device__ int64_t block_sum64(int64_t x, int64_t* scratch /* >= kPlanThreads/64 */) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <class T>
+__device__ __forceinline__ T block_sum(T x, T* scratch /* kPlanWaves */) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-  if (lane == 0) scratch[wave] = x;
+  if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = x;
   __syncthreads();
-  int64_t t = 0;
+  T t = 0;
 #pragma unroll
-  for (int w = 0; w < kPlanThreads / 64; ++w) t += scratch[w];
-  __syncthreads();
+  for (int w = 0; w < kPlanWaves; ++w) t += scratch[w];
   return t;
 }
 
 // The plan of karpo_attn.h from the device bounds, in three passes over the tiles: the pack's workgroup-steps (which
 // set the split length), a histogram of part costs, and the scatter (descending cost order; split tiles' slots and
 // merge entries in tile order). The host planner (plan.cpp) lists the same items; among equal costs the order here
-// depends on atomics. Workgroup b plans job b (the backward's two work lists in one launch).
+// depends on atomics. Workgroup b plans job b (the backward's two work lists in one launch). It is bound by its chain of
+// barriers and dependent loads, so the bounds of up to kPlanSeqs sequences are read once, into LDS, with the tile bases
+// that every tile's search reads; the first 1,024 tiles' places stay in registers between the passes; the divisions are
+// 32-bit; and the scans of the last pass run only when a tile splits. Kernel time of the Qwen pack's plan 10.8 -> 7.8 us
+// (10.7 -> 7.7 us for the backward's two).
 struct PlanJobs {
   PlanJob a, b;
 };
@@ -1230,9 +1235,12 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanJobs jobs, int n
   const int tiles_cap = job.tiles, merges_cap = job.merges, items_cap = job.items;
   int32_t* __restrict__ tile_base = job.tile_base;
   __shared__ int hist[kCostBuckets];
-  __shared__ int scratch[kPlanThreads / 64 + 1];
-  __shared__ int64_t scratch64[kPlanThreads / 64];
+  __shared__ int seqs_s[kPlanSeqs][3];  // per sequence: first tile, query rows, key rows
+  __shared__ int scan_s[3][kPlanWaves];
+  __shared__ int64_t sum_s[2][kPlanWaves];
   const int tid = threadIdx.x;
+  const bool local = n_seq <= kPlanSeqs;
+  for (int b = tid; b < kCostBuckets; b += kPlanThreads) hist[b] = 0;
   // the header's constant entries (an empty plan until the items are listed)
   if (tid == 0) {
     plan[0] = 0;
@@ -1248,60 +1256,71 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanJobs jobs, int n
     plan[10] = g.shape;
     plan[11] = 0;
   }
-  if (job.status != nullptr) {  // the bounds against the call's contract: a violation plans nothing
-    int bad = 0;
-    for (int i = tid; i < n_seq; i += kPlanThreads) {
-      const int q0 = q_cu[i], q1 = q_cu[i + 1], k0 = k_cu[i], k1 = k_cu[i + 1];
-      bad |= q0 < 0 || k0 < 0 || q1 < q0 || k1 < k0 || q1 - q0 > job.max_q || (int64_t)q1 > job.total_q ||
-             (job.key_bound > 0 && (int64_t)k1 > job.key_bound);
-    }
-    int total;
-    block_exclusive_scan(bad, &total, scratch);
-    if (tid == 0) *job.status = total > 0 ? KARPO_ATTN_ERR_BOUNDS : KARPO_ATTN_OK;
-    if (total > 0) return;
-  }
+  int bad = 0;  // the bounds against the call's contract: a violation plans nothing
   int carry = 0;
   for (int base = 0; base < n_seq; base += kPlanThreads) {
     const int i = base + tid;
-    const int nt = i < n_seq ? (int)tiles_of(q_cu[i + 1] - q_cu[i], g.rows) : 0;
+    int nt = 0;
+    if (i < n_seq) {
+      const int q0 = q_cu[i], q1 = q_cu[i + 1], k0 = k_cu[i], k1 = k_cu[i + 1];
+      if (job.status != nullptr)
+        bad |= q0 < 0 || k0 < 0 || q1 < q0 || k1 < k0 || q1 - q0 > job.max_q || (int64_t)q1 > job.total_q ||
+               (job.key_bound > 0 && (int64_t)k1 > job.key_bound);
+      nt = q1 > q0 ? (int)(((uint32_t)(q1 - q0) + (uint32_t)g.rows - 1) / (uint32_t)g.rows) : 0;  // tiles_of
+      if (local) {
+        seqs_s[i][1] = q1 - q0;
+        seqs_s[i][2] = k1 - k0;
+      }
+    }
     int total;
-    const int ex = block_exclusive_scan(nt, &total, scratch);
-    if (i < n_seq) tile_base[i] = carry + ex;
+    const int ex = block_exclusive_scan(nt, &total, scan_s[(base / kPlanThreads) & 1]);
+    if (i < n_seq) {
+      if (local) seqs_s[i][0] = carry + ex;
+      else tile_base[i] = carry + ex;
+    }
     carry += total;
   }
-  if (tid == 0) tile_base[n_seq] = carry;
+  if (job.status != nullptr) {
+    const int any = __syncthreads_or(bad);
+    if (tid == 0) *job.status = any ? KARPO_ATTN_ERR_BOUNDS : KARPO_ATTN_OK;
+    if (any) return;
+  } else {
+    __syncthreads();
+  }
   const int n_tiles = min(carry, tiles_cap);
-  for (int b = tid; b < kCostBuckets; b += kPlanThreads) hist[b] = 0;
-  __syncthreads();
 
   // tile f: its segment, index in the segment and key steps
   auto locate = [&](int f, int* seg, int* t) -> int64_t {
     int l0 = 0, l1 = n_seq;  // last segment whose first tile is at or before f
     while (l1 - l0 > 1) {
       const int mid = (l0 + l1) >> 1;
-      if (tile_base[mid] <= f) l0 = mid; else l1 = mid;
+      if ((local ? seqs_s[mid][0] : tile_base[mid]) <= f) l0 = mid; else l1 = mid;
     }
     *seg = l0;
-    *t = f - tile_base[l0];
-    const int lq = q_cu[l0 + 1] - q_cu[l0], lk = k_cu[l0 + 1] - k_cu[l0];
+    *t = f - (local ? seqs_s[l0][0] : tile_base[l0]);
+    const int lq = local ? seqs_s[l0][1] : q_cu[l0 + 1] - q_cu[l0];
+    const int lk = local ? seqs_s[l0][2] : k_cu[l0 + 1] - k_cu[l0];
     return tile_steps(lq, lk, *t, g.rows, g.bn, left, right);
   };
-  int64_t mine = 0;
-  for (int f = tid; f < n_tiles; f += kPlanThreads) {
+  int seg0 = 0, t0 = 0;  // this thread's tile of the first 1,024
+  int64_t steps0 = 0;
+  if (tid < n_tiles) steps0 = locate(tid, &seg0, &t0);
+  int64_t mine = steps0;
+  for (int f = tid + kPlanThreads; f < n_tiles; f += kPlanThreads) {
     int seg, t;
     mine += locate(f, &seg, &t);
   }
-  const int64_t tau = split_tau(block_sum64(mine, scratch64) * g.n_hg, g.conc);
+  const int64_t tau = split_tau(block_sum(mine, sum_s[0]) * g.n_hg, g.conc);
 
   int64_t counts = 0;  // split tiles (high 32 bits) and items (low) of this thread's tiles
   for (int f = tid; f < n_tiles; f += kPlanThreads) {
     int seg, t;
-    const int64_t steps = locate(f, &seg, &t);
+    const int64_t steps = f < kPlanThreads ? steps0 : locate(f, &seg, &t);
     const int parts = split_parts(steps, tau);
     atomicAdd(&hist[part_cost(steps, parts)], parts);
     counts += (parts > 1 ? (int64_t)1 << 32 : 0) + parts;
   }
-  const int64_t both = block_sum64(counts, scratch64);
+  const int64_t both = block_sum(counts, sum_s[1]);
   // within the capacities by the split policy's bound; a plan that would not fit lists no items (never written)
   const int n_merges = (int)(both >> 32), n_items = (int)(both & 0xffffffff);
   const bool fits = n_merges <= merges_cap && n_items <= items_cap;
@@ -1316,7 +1335,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanJobs jobs, int n
       s += h[r];
     }
     int total;
-    int ex = block_exclusive_scan(s, &total, scratch);
+    int ex = block_exclusive_scan(s, &total, scan_s[2]);
 #pragma unroll
     for (int r = 0; r < per; ++r) {
       hist[kCostBuckets - 1 - (tid * per + r)] = ex;
@@ -1327,18 +1346,23 @@ __global__ __launch_bounds__(kPlanThreads) void plan_kernel(PlanJobs jobs, int n
   int slot_carry = 0, merge_carry = 0;
   for (int base = 0; base < n_tiles; base += kPlanThreads) {
     const int f = base + tid;
-    int seg = 0, t = 0, parts = 0;
-    int64_t steps = 0;
+    int seg = seg0, t = t0, parts = 0;
+    int64_t steps = steps0;
     if (f < n_tiles) {
-      steps = locate(f, &seg, &t);
+      if (base > 0) steps = locate(f, &seg, &t);
       parts = split_parts(steps, tau);
     }
     const bool split = parts > 1;
-    int slots_total, merges_total;
-    const int slot = slot_carry + block_exclusive_scan(split ? parts : 0, &slots_total, scratch);
-    const int merge = merge_carry + block_exclusive_scan(split ? 1 : 0, &merges_total, scratch);
-    slot_carry += slots_total;
-    merge_carry += merges_total;
+    int slot = -1, merge = 0;
+    if (n_merges > 0) {  // slots and merge entries in tile order (parts in the high bits: fewer than 2^31 slots)
+      int64_t total;
+      const int64_t ex = block_exclusive_scan(split ? ((int64_t)parts << 32) + 1 : (int64_t)0, &total,
+                                              sum_s[(base / kPlanThreads) & 1]);
+      slot = slot_carry + (int)(ex >> 32);
+      merge = merge_carry + (int)(ex & 0xffffffff);
+      slot_carry += (int)(total >> 32);
+      merge_carry += (int)(total & 0xffffffff);
+    }
     if (f >= n_tiles || !fits) continue;
     if (split) {
       int32_t* m = plan + kPlanHeader + kMergeInts * merge;

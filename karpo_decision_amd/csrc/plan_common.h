@@ -148,7 +148,8 @@ KA_HD inline int64_t tile_steps(int lq, int lk, int64_t t, int rows, int bn, int
   const int64_t lo = left < 0 ? 0 : ka_max(0, p0 + delta - left);
   const int64_t hi = right < 0 ? (int64_t)lk : ka_min((int64_t)lk, p1 + delta + right + 1);
   if (hi <= lo) return 0;
-  return (hi + bn - 1) / bn - lo / bn;
+  // 32-bit divisions (0 <= lo < hi <= lk): the 64-bit ones are long instruction sequences on the device planner's chain
+  return (int64_t)(((uint32_t)hi + (uint32_t)bn - 1) / (uint32_t)bn) - (int64_t)((uint32_t)lo / (uint32_t)bn);
 }
 
 KA_HD inline int64_t tiles_of(int64_t lq, int rows) { return lq <= 0 ? 0 : (lq + rows - 1) / rows; }
@@ -161,10 +162,12 @@ KA_HD inline int64_t split_tau(int64_t total, int conc) {
   const int64_t tau = (total + conc - 1) / conc;
   return tau < kMinSplitSteps ? kMinSplitSteps : tau;
 }
-KA_HD inline int split_parts(int64_t steps, int64_t tau) { return steps > tau ? (int)((steps + tau - 1) / tau) : 1; }
+KA_HD inline int split_parts(int64_t steps, int64_t tau) {  // steps: at most 2^31 keys' steps
+  return steps > tau ? (int)(((uint32_t)steps + (uint32_t)tau - 1) / (uint32_t)tau) : 1;
+}
 // Ordering cost of one part of a tile: its steps, plus one for the store (clamped to the histogram).
 KA_HD inline int part_cost(int64_t steps, int parts) {
-  const int64_t c = (steps + parts - 1) / parts + 1;
+  const int64_t c = (int64_t)(((uint32_t)steps + (uint32_t)parts - 1) / (uint32_t)parts) + 1;
   return (int)ka_min(c, kCostBuckets - 1);
 }
 // Partial slots (per head group) the parts of split tiles can take, and the split tiles there can be.
