@@ -412,6 +412,7 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
   const uint16_t* kbase = p.k + (int64_t)kvh * p.sk_h + (GATHER ? 0 : (int64_t)ka * p.sk_t);
   const uint16_t* vbase = p.v + (int64_t)kvh * p.sv_h + (GATHER ? 0 : (int64_t)ka * p.sv_t);
   constexpr int GI = GATHER ? INSTS : 1;
+  constexpr bool V_LAYOUT = D == 512 || (SHAPE == kNarrow && !GATHER);
   uint32_t k_voff[INSTS], v_voff[INSTS];
   int k_key[GI], v_key[GI], k_row[GI], v_row[GI];
 #pragma unroll
@@ -424,7 +425,8 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
     } else {
       k_voff[r] = (uint32_t)(key * p.sk_t + colm) * 2u;
     }
-    v_dma_source<D>(wave * INSTS + r, lane, &key, &colm);
+    if constexpr (V_LAYOUT) v_layout_source<D>(wave * INSTS + r, lane, &key, &colm);
+    else v_dma_source<D>(wave * INSTS + r, lane, &key, &colm);
     if constexpr (GATHER) {
       v_key[r] = key;
       v_voff[r] = (uint32_t)colm * 2u;
@@ -487,8 +489,11 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
   const int k_read[2] = {s_offset<D>(key_row(col), half) + dh * QC * 512,
                          s_offset<D>(key_row(col), 2 + half) + dh * QC * 512};
   const int g = lane >> 4, jl = lane & 15;
-  const int v_read =
-      v_offset<D>(8 * (g >> 1) + (jl >> 2), 16 * (g & 1) + 4 * (jl & 3)) + dh * OB * 256;  // + kc, rr, db offsets
+  // V transposed, four rows of 32 columns per read rr: v_read[rr] + kc * V_KC + db * V_DB
+  constexpr int V_KC = V_LAYOUT ? (D / 16) * 512 : (D / 8) * 256, V_DB = V_LAYOUT ? 256 : 1024;
+  const int v_first = v_offset<D>(8 * (g >> 1) + (jl >> 2), 16 * (g & 1) + 4 * (jl & 3)) + dh * OB * 256;
+  const int v_read[2] = {V_LAYOUT ? v_first : s_tr_base(lane, 0),
+                         V_LAYOUT ? v_first + (D / 16) * 128 : s_tr_base(lane, 1)};
 
   f32x16 acc[QB][OB];
 #pragma unroll
@@ -660,7 +665,7 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
           for (int rr = 0; rr < 2; ++rr)
             pv[rr] = __builtin_bit_cast(
                 bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                            (KA_LDS s16x4*)(vt + v_read + (kc * 4 + rr) * (D / 16) * 128 + db * 256)));
+                            (KA_LDS s16x4*)(vt + v_read[rr] + kc * V_KC + db * V_DB)));
           const bf16x8 a = __builtin_shufflevector(pv[0], pv[1], 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
           for (int b = 0; b < QB; ++b)  // one V operand read feeds every query block

@@ -28,8 +28,9 @@ constexpr int kBufferFlags = 0x00020000;
 // Row of the 32-key block that MFMA A-row r reads: bits 2 and 3 of r swapped.
 __device__ __forceinline__ int key_row(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
 
-// Byte offset inside the forward's V tile: (key k, element d) at
-// ((k / 4) * D/16 + d / 16) * 128 + (k % 4) * 32 + (d % 16) * 2. Its K tile is in the S layout (s_offset).
+// Byte offset inside the V layout (the forward's V tiles at head size 512 and in streaming one-wave tiles): (key k,
+// element d) at
+// ((k / 4) * D/16 + d / 16) * 128 + (k % 4) * 32 + (d % 16) * 2. The other K and V tiles are in the S layout (s_offset).
 template <int D>
 __device__ __forceinline__ int v_offset(int k, int d) {
   return ((k >> 2) * (D / 16) + (d >> 4)) * 128 + (k & 3) * 32 + (d & 15) * 2;

@@ -18,13 +18,23 @@ KA_HD inline void k_dma_source(int blk, int lane, int* key, int* col) {
   *key = (blk / (D / 32)) * 16 + (lane >> 2);
   *col = (blk % (D / 32)) * 32 + ((lane & 3) ^ (lane >> 4)) * 8;
 }
-// The same for the V tile (the inverse of v_offset): two consecutive lanes read 32 consecutive bytes.
+// The V layout (v_offset, mfma_common.h): two consecutive lanes read 32 consecutive bytes, an instruction 256 bytes of
+// each of four keys.
 template <int D>
-KA_HD inline void v_dma_source(int blk, int lane, int* key, int* col) {
+KA_HD inline void v_layout_source(int blk, int lane, int* key, int* col) {
   const int b = blk * 8 + (lane >> 3);  // 128-byte block: (key group, d block)
   const int piece = lane & 7;
   *key = (b / (D / 16)) * 4 + (piece >> 1);
   *col = (b % (D / 16)) * 16 + (piece & 1) * 8;
+}
+// The V tile's copies: the K tile's layout, or the V layout at head size 512 (its reads need one base register instead
+// of two, and the pair tiles have none to spare). One-wave tiles that stream their keys from HBM keep the V layout too,
+// which reads the same chunks of the same keys in another order: 64 B of a key per instruction took the markers layer
+// from 121 to 132 us (half a cache line per request, streamed past the caches).
+template <int D>
+KA_HD inline void v_dma_source(int blk, int lane, int* key, int* col) {
+  if (D < 512) k_dma_source<D>(blk, lane, key, col);
+  else v_layout_source<D>(blk, lane, key, col);
 }
 
 // The tile vector that lane column `col` (0-31) of wave `wave` holds in its query block `block`: a wave's blocks (a
