@@ -13,8 +13,8 @@ LIBRARY = Path(__file__).resolve().parent / "libkarpo_attn.so"
 #: Every symbol ``include/karpo_attn.h`` declares.
 EXPORTS = ("karpo_attn_fwd", "karpo_attn_plan", "karpo_attn_plan_capacity", "karpo_attn_workspace_bytes",
            "karpo_attn_tile_shape", "karpo_attn_strerror", "karpo_attn_version", "karpo_attn_norm_rope",
-           "karpo_attn_bwd_workspace_bytes", "karpo_attn_bwd_workspace_best_bytes", "karpo_attn_bwd", "karpo_attn_device_status",
-           "karpo_attn_fwd_noalloc")
+           "karpo_attn_bwd_workspace_bytes", "karpo_attn_bwd_workspace_best_bytes", "karpo_attn_bwd",
+           "karpo_attn_device_status", "karpo_attn_fwd_noalloc")
 
 OK = 0
 ERR_HEAD_DIM, ERR_HEADS, ERR_LAYOUT, ERR_WINDOW, ERR_SPANS, ERR_ARG, ERR_BOUNDS = 2, 3, 4, 6, 7, 9, 11

@@ -8,15 +8,15 @@
 // MFMA rate), and it computes S and dP twice (seven products). P and dS cost 10 bytes of traffic per visible pair and
 // 5,120 FLOPs need them, so keeping them takes less time than either the recomputation or the exchange: five products,
 // each a plain tiled matrix product with every accumulator in one wave's registers. Measured against the wave pairs
-// (32 / 4 heads, causal, MI355X): 497 -> 140 us at 512 rows, 2.09 -> 0.83 ms at 2,048, 12.4 -> 8.0 ms at 8,192, 48.1 ->
-// 24.4 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
+// (32 / 4 heads, causal, MI355X): 427 -> 121 us at 512 rows, 1.79 -> 0.64 ms at 2,048, 10.6 -> 6.1 ms at 8,192, 48.1 ->
+// 23.2 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
 // call takes this path when the workspace has room for a chunk of 256 rows.
 //
 // P and dS in the workspace: per head [key block of 16][chunk of 8 rows][16 keys][8 rows] bf16, the 16 keys of a
 // 256-byte run XOR-swizzled by the chunk index (key ^ 4 (chunk % 4): free of bank conflicts read either way), the layout
-// in which a tile is read from LDS: a copy instruction moves 1 KiB of consecutive bytes. A lane of kernel 1 holds one key's scores of 8
-// consecutive rows (the MFMA's A rows are taken in key_row order) and stores them as one 16-byte chunk; dK and dV read
-// those chunks directly as MFMA operands, dQ reads the same tile transposed.
+// in which a tile is read from LDS: a copy instruction moves 1 KiB of consecutive bytes. A lane of kernel 1 holds one
+// key's scores of 8 consecutive rows (the MFMA's A rows are taken in key_row order) and stores them as one 16-byte
+// chunk; dK and dV read those chunks directly as MFMA operands, dQ reads the same tile transposed.
 //
 // Chunks of rows run in ascending order. dQ of a chunk's rows is complete within it; dK and dV go on from one chunk to
 // the next in fp32 (workspace, in the accumulators' register order) and are rounded once, in the last chunk.
@@ -506,9 +506,17 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_wide_grad_kernel(BwdWideP
   KA_LDS char* const at[kRing] = {(KA_LDS char*)a0_s, (KA_LDS char*)a1_s, (KA_LDS char*)a2_s, (KA_LDS char*)a3_s};
   KA_LDS char* const bt[kRing] = {(KA_LDS char*)b0_s, (KA_LDS char*)b1_s, (KA_LDS char*)b2_s, (KA_LDS char*)b3_s};
   const WideSeq s(w);
+  // dK and dV first where the group is large: their items are then the longer ones (rows / 32 steps of every head of the
+  // group, against the visible keys / 32 of dQ), and early chunks have few of them, so dQ fills the CUs that they leave
+  // free. Backward at 32 / 4 heads: 697 -> 637 us at 2,048 rows, 1.91 -> 1.80 ms at 4,096, 6.21 -> 6.11 at 8,192; at
+  // 32 / 16 heads (group 2) 1-2% slower at 4,096 and 8,192 rows.
+  const int dkdv_items = w.keys / kGradTile * 4 * (w.b.heads / w.b.group);
   const int dq_items = w.rows / kGradTile * 2 * w.b.heads;
-  if ((int)blockIdx.x < dq_items) wide_grad<true>(w, s, blockIdx.x, at, bt);
-  else wide_grad<false>(w, s, blockIdx.x - dq_items, at, bt);
+  const bool dkdv_first = w.b.group >= 4;
+  const int at_dkdv = (int)blockIdx.x - (dkdv_first ? 0 : dq_items);
+  const int at_dq = (int)blockIdx.x - (dkdv_first ? dkdv_items : 0);
+  if (at_dkdv >= 0 && at_dkdv < dkdv_items) wide_grad<false>(w, s, at_dkdv, at, bt);
+  else wide_grad<true>(w, s, at_dq, at, bt);
 }
 
 hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream) {
@@ -518,7 +526,8 @@ hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream) {
   const int64_t per = row_tiles * key_tiles / 1024;
   w.run = (int32_t)(per < 1 ? 1 : per > 8 ? 8 : per);
   const int64_t ds_items = row_tiles * ((key_tiles + w.run - 1) / w.run);
-  const int64_t grad_items = (int64_t)(w.rows / kGradTile) * 2 * w.b.heads + (int64_t)(w.keys / kGradTile) * 4 * kv_heads;
+  const int64_t grad_items =
+      (int64_t)(w.rows / kGradTile) * 2 * w.b.heads + (int64_t)(w.keys / kGradTile) * 4 * kv_heads;
   for (int64_t r = 0; r < w.b.total_q; r += w.rows) {
     w.r_begin = (int32_t)r;
     hipLaunchKernelGGL(bwd_wide_ds_kernel, dim3((unsigned)ds_items), dim3(kWideThreads), 0, stream, w);
