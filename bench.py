@@ -247,7 +247,7 @@ def backward(args, device, w) -> int:
                    "flops_per_step": flops, "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4), "traffic": None,
-                     "kernel": (f"karpo_attn_bwd (bwd_stats_kernel, bwd_dq_pair_kernel<512>, bwd_dkdv_pair_kernel<512>)"
+                     "kernel": (f"karpo_attn_bwd (bwd_stats_kernel<512>, bwd_wide_ds_kernel, bwd_wide_grad_kernel)"
                                 if w.head_dim == 512 else
                                 f"karpo_attn_bwd (bwd_dq_kernel<{w.head_dim}>, "
                                 f"bwd_dkdv_kernel<{w.head_dim}, *>)"),
