@@ -187,7 +187,9 @@ typedef struct KarpoAttnBwdArgs {
 /* The least workspace the call runs in, and the workspace its fastest path takes (never less; the same for most
  * calls). At head size 512 a call of one sequence without a left window bound or spans holds P and dS of a chunk of
  * query rows (at most 4 GiB) and, over several chunks, dK and dV in fp32; karpo_attn_bwd takes that path when
- * workspace_bytes allows it, and the path of the least workspace otherwise. */
+ * workspace_bytes has room for chunks long enough to be faster (256 to 8,192 rows, by the head counts and the number
+ * of chunks), and the path of the least workspace otherwise. The path and its chunks set the order of the fp32 sums:
+ * calls are bitwise equal for equal arguments, workspace_bytes among them. */
 int karpo_attn_bwd_workspace_bytes(const KarpoAttnBwdArgs* args, size_t* bytes);
 int karpo_attn_bwd_workspace_best_bytes(const KarpoAttnBwdArgs* args, size_t* bytes);
 int karpo_attn_bwd(const KarpoAttnBwdArgs* args, void* stream);

@@ -356,8 +356,25 @@ struct WideSizes {
   int64_t rows, keys, p_offset, ds_offset, acc_offset, bytes;
 };
 
-constexpr int64_t kWideBytes = (int64_t)4 << 30;  // P and dS of one chunk at most
+// P and dS of one chunk at most. 32 / 4 heads, causal, with 1, 2, 4, 8 GiB: 27.5, 23.5, 22.9, 22.5 ms at 16,384 rows, 141,
+// 106, 90.5, 90.8 ms at 32,768; 32 / 16 heads 32.5, 27.6, 25.9, 24.9 and 157, 124, 107, 103 ms.
+constexpr int64_t kWideBytes = (int64_t)4 << 30;
 constexpr int64_t kWideTile = 256;
+
+// Whether chunks of `rows` query rows are faster than the wave pairs (one chunk always is). Every chunk but the last
+// writes, and every one but the first reads, dK and dV of its keys in fp32, which rows * group query rows of products
+// per key have to pay for; and a chunk's dQ tiles each walk all visible keys, so where a chunk is too small to fill the GPU
+// the chunks' walks add up, against one walk of the group's rows in the pairs. Wave pairs against chunks, causal:
+//   16,384 rows, 32 / 32 heads: 42.9 ms; of 256 rows 57.2, 512 42.3, 1,024 33.5      (4,096 rows: 2.88; 4.05, 2.99, 2.41)
+//                32 / 16: 41.3; 40.7, 32.5, 27.5                                     (4,096 rows: 2.86; 2.99, 2.36, 1.96)
+//                32 / 8:  40.7; 41.1, 30.8, 24.6      32 / 4: 41.1; 35.3, 27.6, 23.6      8 / 1: 16.7; 15.4, 10.7, 8.0
+//                8 / 8:   10.6; of 1,024 rows 8.4     4 / 4: 5.4; 5.7, of 2,048 4.0       2 / 2: 2.7; 4.1, 2.8
+//   65,536 rows, 1 / 1 head: 20.6; of 2,048 rows 32.3, 16,384 13.1                    4 / 1: 82; of 1,024 rows 89, 2,048 63
+//   131,072 rows, 32 / 4: 2,626; of 256 rows 2,176
+bool wide_chunks_pay(int64_t rows, int64_t chunks, int64_t heads, int64_t group) {
+  const int64_t least = group >= 8 ? 256 : group >= 2 ? 512 : 1024;
+  return chunks == 1 || (rows >= least && (rows * heads >= 8192 || chunks <= 6 * group));
+}
 
 // The largest chunks that `limit` bytes of workspace hold (SIZE_MAX: the path's own choice).
 WideSizes wide_sizes_of(const KarpoAttnBwdArgs* b, const BwdSizes& z, size_t limit) {
@@ -378,6 +395,7 @@ WideSizes wide_sizes_of(const KarpoAttnBwdArgs* b, const BwdSizes& z, size_t lim
     chunks = (all + most - 1) / most;
   }
   const int64_t rows = ((all + chunks - 1) / chunks + kWideTile - 1) / kWideTile * kWideTile;
+  if (!wide_chunks_pay(rows, chunks, a->heads, a->heads / a->kv_heads)) return w;
   if ((rows / 256) * (keys / 128) * a->heads > INT32_MAX ||
       (rows / 256) * 2 * a->heads + (keys / 256) * 4 * a->kv_heads > INT32_MAX)
     return w;

@@ -347,6 +347,24 @@ def test_bwd_workspace_holds_stats_and_both_plans():
     assert lib.karpo_attn_bwd(ctypes.byref(_bwd_args(_args(total_q=0, total_k=100))), None) == 0  # nothing to do
 
 
+@pytest.mark.parametrize("heads,kv_heads,rows,chunked", [
+    (32, 4, 16384, True), (32, 4, 131072, True),   # group 8: from 256 rows a chunk
+    (32, 16, 65536, True),                         # group 2: chunks of 512 rows
+    (32, 32, 32768, True), (32, 32, 65536, False),  # group 1: chunks of 1,024 rows, of 512
+    (1, 1, 65536, True), (1, 1, 4096, True),       # four chunks of 16,384 rows, one chunk
+    (8, 4, 262144, False),                         # group 2: chunks of 512 rows that leave the GPU idle, 512 of them
+])
+def test_bwd_chunks_only_where_they_are_faster(heads, kv_heads, rows, chunked):
+    """Head size 512, one sequence: the workspace of the chunked path (4 GiB of P and dS at most) only where its chunks
+    are longer than those that lose to the wave pairs."""
+    lib = _lib.load()
+    b = _bwd_args(_args(n_seq=1, heads=heads, kv_heads=kv_heads, head_dim=512, total_q=rows, max_q=rows, total_k=rows))
+    least, best = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(least)) == 0
+    assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(best)) == 0
+    assert (best.value > least.value) == chunked, (least.value, best.value)
+
+
 def test_empty_pack_is_a_no_op():
     lib = _lib.load()
     assert lib.karpo_attn_fwd(ctypes.byref(_args(total_q=0)), None) == 0
