@@ -444,6 +444,41 @@ def _workspace(lib, fn, args, device: torch.device) -> Tensor:
     return torch.empty(need.value, dtype=torch.uint8, device=device)
 
 
+def _free_bytes(device: torch.device) -> int | None:
+    """Bytes the device could still give this process (free, or free in torch's cache); None during a graph capture."""
+    if torch.cuda.is_current_stream_capturing():
+        return None
+    stats = torch.cuda.memory_stats_as_nested_dict(device)
+    cached = stats["reserved_bytes"]["all"]["current"] - stats["allocated_bytes"]["all"]["current"]
+    return torch.cuda.mem_get_info(device)[0] + cached
+
+
+#: Workspaces from which a backward first asks what the device has (10 us; such calls take 300 us and more).
+_LARGE = 1 << 28
+
+
+def _backward_workspace(lib, args, device: torch.device) -> Tensor:
+    """The workspace of the backward's fastest path (``karpo_attn_bwd_workspace_best_bytes``: at head size 512 up to
+    4 GiB of scores, and dK / dV in fp32), or where the device has not got it the largest of its half, quarter, ... down
+    to the least (``karpo_attn_bwd`` then takes shorter chunks, or the path that keeps no scores). A size above what the
+    device has left is not asked for: each such request would make torch's allocator give back its whole cache. The
+    workspace sets the order of the fp32 sums, so gradients are bitwise repeatable while the same size is to be had."""
+    least, best = ctypes.c_size_t(), ctypes.c_size_t()
+    _lib.check(lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(args), ctypes.byref(least)), "packed attention backward")
+    _lib.check(lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(args), ctypes.byref(best)),
+               "packed attention backward")
+    size = best.value
+    free = _free_bytes(device) if size >= _LARGE else None
+    while size > least.value:
+        if free is None or size <= free:
+            try:
+                return torch.empty(size, dtype=torch.uint8, device=device)
+            except torch.OutOfMemoryError:
+                pass
+        size //= 2
+    return torch.empty(least.value, dtype=torch.uint8, device=device)
+
+
 @torch.library.custom_op(f"{NAMESPACE}::packed_attention_lse", mutates_args=())
 def packed_attention_lse(query: Tensor, key: Tensor, value: Tensor, q_cu: Tensor, k_cu: Tensor, max_q: int,
                          scale: float, window_left: int, window_right: int,
@@ -507,13 +542,9 @@ def packed_attention_backward(grad: Tensor, query: Tensor, key: Tensor, value: T
         b.d_q, b.d_q_stride_tok, b.d_q_stride_head = dq.data_ptr(), dq.stride(0), dq.stride(1)
         b.d_k, b.d_k_stride_tok, b.d_k_stride_head = dk.data_ptr(), dk.stride(0), dk.stride(1)
         b.d_v, b.d_v_stride_tok, b.d_v_stride_head = dv.data_ptr(), dv.stride(0), dv.stride(1)
-        workspace = None
-        if query.shape[2] == 512:  # the workspace of the fastest path where the device has it
-            try:
-                workspace = _workspace(lib, lib.karpo_attn_bwd_workspace_best_bytes, b, query.device)
-            except torch.OutOfMemoryError:
-                pass
-        if workspace is None:
+        if query.shape[2] == 512:
+            workspace = _backward_workspace(lib, b, query.device)
+        else:
             workspace = _workspace(lib, lib.karpo_attn_bwd_workspace_bytes, b, query.device)
         b.fwd.workspace, b.fwd.workspace_bytes = workspace.data_ptr(), workspace.numel()
         stream = _current_stream(query.device.index)

@@ -344,7 +344,7 @@ def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, k
     chunk = -(-heads * 2 * (lq + pad) * 4 // 256) * 256 + 4 * 256 * keys * heads + 2 * keys * kv_heads * 512 * 4
     got = {}
     for form in ("least", "chunks", "best"):
-        def workspace(lib, fn, args, device):
+        def workspace(lib, args, device):
             least, best = ctypes.c_size_t(), ctypes.c_size_t()
             assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(args), ctypes.byref(least)) == 0
             assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(args), ctypes.byref(best)) == 0
@@ -352,7 +352,7 @@ def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, k
             assert best.value >= size or form == "chunks"
             return torch.full((size,), 255, dtype=torch.uint8, device=device)
 
-        monkeypatch.setattr(ops, "_workspace", workspace)
+        monkeypatch.setattr(ops, "_backward_workspace", workspace)
         print("head 512 one sequence", (lq, lk), form, flush=True)
         got[form] = ops.packed_attention_backward(do, q, k, v, out, lse, qc, kc, lq, 0.05, -1, right, None)
         torch.cuda.synchronize()

@@ -365,6 +365,39 @@ def test_bwd_chunks_only_where_they_are_faster(heads, kv_heads, rows, chunked):
     assert (best.value > least.value) == chunked, (least.value, best.value)
 
 
+@pytest.mark.parametrize("room,free,steps", [
+    (1 << 40, 1 << 40, [1]),               # the fastest path's workspace
+    (3 << 30, 1 << 40, [1, 2]),            # refused once (4.3 GiB), then half of it
+    (3 << 30, 3 << 30, [2]),               # not asked for where the device is known not to have it
+    (700 << 20, 1 << 30, [8]),
+    (200 << 20, None, [1, 2, 4, 8, 16, 32]),  # under capture: tried, each refusal halves it
+    (40 << 20, 40 << 20, [128]),           # too little for a chunk of 256 rows, still above the least
+    (4_400_000, 4_400_000, [0]),           # the least
+])
+def test_bwd_workspace_when_memory_is_short(monkeypatch, room, free, steps):
+    """16,384 rows of 32 / 4 heads at head size 512: the allocations that the backward tries (as divisors of the best
+    size, 0: the least), with `room` bytes to be had and `free` reported; the largest that fits is returned."""
+    lib = _lib.load()
+    rows = 16384
+    b = _bwd_args(_args(n_seq=1, heads=32, kv_heads=4, head_dim=512, total_q=rows, max_q=rows, total_k=rows))
+    least, best = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(least)) == 0
+    assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(best)) == 0
+    assert least.value < 5 << 20 and best.value > 4 << 30
+    asked = []
+
+    def empty(size, dtype, device):
+        asked.append(size)
+        if size > room:
+            raise torch.OutOfMemoryError("no room")
+        return torch.zeros(0, dtype=dtype)
+
+    monkeypatch.setattr(ops, "_free_bytes", lambda device: free)
+    monkeypatch.setattr(ops.torch, "empty", empty)
+    ops._backward_workspace(lib, b, torch.device("cpu"))
+    assert asked == [best.value // s if s else least.value for s in steps]
+
+
 def test_empty_pack_is_a_no_op():
     lib = _lib.load()
     assert lib.karpo_attn_fwd(ctypes.byref(_args(total_q=0)), None) == 0
