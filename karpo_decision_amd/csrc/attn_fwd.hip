@@ -412,7 +412,7 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
   const uint16_t* kbase = p.k + (int64_t)kvh * p.sk_h + (GATHER ? 0 : (int64_t)ka * p.sk_t);
   const uint16_t* vbase = p.v + (int64_t)kvh * p.sv_h + (GATHER ? 0 : (int64_t)ka * p.sv_t);
   constexpr int GI = GATHER ? INSTS : 1;
-  constexpr bool V_LAYOUT = D == 512 || (SHAPE == kNarrow && !GATHER);
+  constexpr bool V_LAYOUT = v_layout(D, SHAPE, GATHER);
   uint32_t k_voff[INSTS], v_voff[INSTS];
   int k_key[GI], v_key[GI], k_row[GI], v_row[GI];
 #pragma unroll
@@ -425,8 +425,7 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
     } else {
       k_voff[r] = (uint32_t)(key * p.sk_t + colm) * 2u;
     }
-    if constexpr (V_LAYOUT) v_layout_source<D>(wave * INSTS + r, lane, &key, &colm);
-    else v_dma_source<D>(wave * INSTS + r, lane, &key, &colm);
+    v_dma_source<D>(V_LAYOUT, wave * INSTS + r, lane, &key, &colm);
     if constexpr (GATHER) {
       v_key[r] = key;
       v_voff[r] = (uint32_t)colm * 2u;
@@ -911,7 +910,7 @@ __global__ __launch_bounds__(512, 2) void attn_fwd_pair_pp_kernel(Params p) {
     int key, colm;
     k_dma_source<D>(wave * INSTS, lane, &key, &colm);
     k_voff0 = (uint32_t)(key * p.sk_t + colm) * 2u;
-    v_dma_source<D>(wave * INSTS, lane, &key, &colm);
+    v_dma_source<D>(true, wave * INSTS, lane, &key, &colm);
     v_voff0 = (uint32_t)(key * p.sv_t + colm) * 2u;
   }
   // T(t) = K(t), V(t - 1): running pointers, empty ranges past the ends (every wave issues 2 INSTS copies per T)

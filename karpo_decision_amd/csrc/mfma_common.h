@@ -28,14 +28,6 @@ constexpr int kBufferFlags = 0x00020000;
 // Row of the 32-key block that MFMA A-row r reads: bits 2 and 3 of r swapped.
 __device__ __forceinline__ int key_row(int r) { return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1); }
 
-// Byte offset inside the V layout (the forward's V tiles at head size 512 and in streaming one-wave tiles): (key k,
-// element d) at
-// ((k / 4) * D/16 + d / 16) * 128 + (k % 4) * 32 + (d % 16) * 2. The other K and V tiles are in the S layout (s_offset).
-template <int D>
-__device__ __forceinline__ int v_offset(int k, int d) {
-  return ((k >> 2) * (D / 16) + (d >> 4)) * 128 + (k & 3) * 32 + (d & 15) * 2;
-}
-
 // The maximum over a lane and the lane 32 away. IEEE maximum (NaN-propagating): one v_maximum3_f32, where fmaxf would
 // first quiet both swapped values.
 __device__ __forceinline__ float half_swap_max(float x) {
@@ -60,20 +52,7 @@ __device__ __forceinline__ int wave_max(int x) {
   return x;
 }
 
-// The S layout: rows (keys, or query rows) staged once and read both as MFMA row operands (ds_read_b128, one row's
-// 16-byte chunk per lane) and transposed (ds_read_b64_tr_b16, four rows of one column group per lane). 16 rows x 4
-// chunks (64 B) make a 1 KiB block; in it row k's 64 B sit at (k % 16) * 64, its chunks XOR-swizzled by k / 4:
-//   s_offset = ((k / 16) * D/32 + c / 4) * 1024 + (k % 16) * 64 + ((c % 4) ^ (k / 4 % 4)) * 16.
-// The 16 lanes of a row read (16 rows, one chunk) cover 64 distinct banks, and the 32 lanes of a transposed read (four
-// rows x chunks c .. c+3) one contiguous 256 B run. Four consecutive lanes of a copy read 64 consecutive bytes: a
-// copy instruction whose neighbouring lanes read different rows takes the address unit a cycle per lane whatever its
-// total (9.5 TB/s out of L2 over the GPU, against 20-31 for 64 B and 31 for 128 B per row; 1 MiB read by 256
-// workgroups), which bounded the kernels while chunk c of 16 rows made a 256 B run.
-template <int D>
-KA_HD inline int s_offset(int k, int c) {
-  return ((k >> 4) * (D / 32) + (c >> 2)) * 1024 + (k & 15) * 64 + ((c & 3) ^ ((k >> 2) & 3)) * 16;
-}
-// Inverse of s_offset for byte offset blk * 1024 + lane * 16 (the copy's source row and first column).
+// Copies into the S layout (s_offset, tile_addr.h): the source row and first column of the chunk at blk * 1024 + lane * 16.
 template <int D>
 KA_HD inline void s_dma_source(int blk, int lane, int* row, int* col) { k_dma_source<D>(blk, lane, row, col); }
 // A wave's INSTS consecutive blocks (blocks INSTS * wave ..) lie in the same 16 rows, 64 B apart: the byte offset of

@@ -1,5 +1,5 @@
 // Per-lane addressing of the forward kernel (attn_fwd.hip), as host-and-device functions: where each lane's copy
-// instructions read (the DMA sources), which keys a query lane sees, which key steps a part of a tile visits, and the
+// instructions read (the DMA sources) and where a tile's elements sit in LDS, which keys a query lane sees, which key steps a part of a tile visits, and the
 // byte offset of a row read through a row table. The kernel computes every address from these functions; a host
 // replay (tests/replay/fwd_replay.cpp) walks every work item of a plan with the same functions and checks each access
 // against the allocations.
@@ -10,31 +10,49 @@
 
 namespace karpo {
 
+// The S layout: rows (keys, or query rows) staged once and read both as MFMA row operands (ds_read_b128, one row's
+// 16-byte chunk per lane) and transposed (ds_read_b64_tr_b16, four rows of one column group per lane). 16 rows x 4
+// chunks (64 B) make a 1 KiB block; in it row k's 64 B sit at (k % 16) * 64, its chunks XOR-swizzled by k / 4:
+//   s_offset = ((k / 16) * D/32 + c / 4) * 1024 + (k % 16) * 64 + ((c % 4) ^ (k / 4 % 4)) * 16.
+// The 16 lanes of a row read (16 rows, one chunk) cover 64 distinct banks, and the 32 lanes of a transposed read (four
+// rows x chunks c .. c+3) one contiguous 256 B run. Four consecutive lanes of a copy read 64 consecutive bytes: a
+// copy instruction whose neighbouring lanes read different rows takes the address unit a cycle per lane whatever its
+// total (9.5 TB/s out of L2 over the GPU, against 20-31 for 64 B and 31 for 128 B per row; 1 MiB read by 256
+// workgroups), which bounded the kernels while chunk c of 16 rows made a 256 B run.
+template <int D>
+KA_HD inline int s_offset(int k, int c) {
+  return ((k >> 4) * (D / 32) + (c >> 2)) * 1024 + (k & 15) * 64 + ((c & 3) ^ ((k >> 2) & 3)) * 16;
+}
+// The V layout: (key k, element d) at ((k / 4) * D/16 + d / 16) * 128 + (k % 4) * 32 + (d % 16) * 2.
+template <int D>
+KA_HD inline int v_offset(int k, int d) {
+  return ((k >> 2) * (D / 16) + (d >> 4)) * 128 + (k & 3) * 32 + (d & 15) * 2;
+}
+// Whether a tile's V is in the V layout (K and every other V are in the S layout): at head size 512, where its reads
+// need one base register instead of two and the pair tiles have none to spare, and in one-wave tiles that stream their
+// keys from HBM: 64 B of a key per copy instruction instead of 256 took the markers layer from 121 to 132 us (half a
+// cache line per request, streamed past the caches).
+KA_HD constexpr bool v_layout(int head_dim, int shape, bool gather) {
+  return head_dim == 512 || (shape == kNarrow && !gather);
+}
+
 // Where lane `lane` of DMA instruction `blk` (1 KiB of the K tile each: 16 keys x 64 B) reads: the key row inside the
-// step and the element column. The inverse of s_offset (mfma_common.h) for byte offset blk * 1024 + lane * 16: four
-// consecutive lanes read 64 consecutive bytes of one key.
+// step and the element column. The inverse of s_offset for byte offset blk * 1024 + lane * 16: four consecutive lanes
+// read 64 consecutive bytes of one key.
 template <int D>
 KA_HD inline void k_dma_source(int blk, int lane, int* key, int* col) {
   *key = (blk / (D / 32)) * 16 + (lane >> 2);
   *col = (blk % (D / 32)) * 32 + ((lane & 3) ^ (lane >> 4)) * 8;
 }
-// The V layout (v_offset, mfma_common.h): two consecutive lanes read 32 consecutive bytes, an instruction 256 bytes of
-// each of four keys.
+// The same for the V tile, in the V layout (the inverse of v_offset: two consecutive lanes read 32 consecutive bytes, an
+// instruction 256 bytes of each of four keys) or in K's.
 template <int D>
-KA_HD inline void v_layout_source(int blk, int lane, int* key, int* col) {
+KA_HD inline void v_dma_source(bool layout, int blk, int lane, int* key, int* col) {
+  if (!layout) return k_dma_source<D>(blk, lane, key, col);
   const int b = blk * 8 + (lane >> 3);  // 128-byte block: (key group, d block)
   const int piece = lane & 7;
   *key = (b / (D / 16)) * 4 + (piece >> 1);
   *col = (b % (D / 16)) * 16 + (piece & 1) * 8;
-}
-// The V tile's copies: the K tile's layout, or the V layout at head size 512 (its reads need one base register instead
-// of two, and the pair tiles have none to spare). One-wave tiles that stream their keys from HBM keep the V layout too,
-// which reads the same chunks of the same keys in another order: 64 B of a key per instruction took the markers layer
-// from 121 to 132 us (half a cache line per request, streamed past the caches).
-template <int D>
-KA_HD inline void v_dma_source(int blk, int lane, int* key, int* col) {
-  if (D < 512) k_dma_source<D>(blk, lane, key, col);
-  else v_layout_source<D>(blk, lane, key, col);
 }
 
 // The tile vector that lane column `col` (0-31) of wave `wave` holds in its query block `block`: a wave's blocks (a

@@ -4,7 +4,8 @@
 // checks it against the allocations: plan entries and bounds read inside their arrays, query rows and output rows
 // inside the tensors, row-table reads inside the table, every DMA chunk either wholly inside its buffer resource
 // (and that range inside the K / V allocation) or wholly past it without a 32-bit wrap, LDS writes inside the tile,
-// partial writes inside the workspace. It also records which (query row, head) outputs the launch writes, so a
+// partial writes inside the workspace; and each chunk lands where the kernel's operand reads look for its key and
+// elements (s_offset, v_offset). It also records which (query row, head) outputs the launch writes, so a
 // plan that leaves a row of a sequence unwritten, or writes one twice, is reported.
 //
 // Test infrastructure only (built by tests/test_replay.py with the host compiler); it mirrors the kernel's control
@@ -61,6 +62,7 @@ int replay(const Call& c, Report& r, std::vector<uint8_t>& written) {
   const FwdSizes z = fwd_sizes(a->total_q, a->n_seq, a->max_q, D, g);
   const int W = g.waves, BN = g.bn, QB = tile_blocks(D, g.shape);
   const bool pair = D == 512;
+  const bool vl = v_layout(D, g.shape, gather);
   const int NB = kv_buffers(D, g.shape, gather);
   const int TILE = BN * D * 2, BLKS = TILE / 1024, INSTS = (BLKS + W - 1) / W;
   const int V = g.vectors;
@@ -141,7 +143,7 @@ int replay(const Call& c, Report& r, std::vector<uint8_t>& written) {
           for (int lane = 0; lane < 64; ++lane) {
             int kk, vk, col;
             k_dma_source<D>(w * INSTS + ri, lane, &kk, &col);
-            v_dma_source<D>(w * INSTS + ri, lane, &vk, &col);
+            v_dma_source<D>(vl, w * INSTS + ri, lane, &vk, &col);
             const int at = (w * INSTS + ri) * 64 + lane;
             for (int which = 0; which < 2; ++which) {
               const int key = which ? vk : kk;
@@ -178,7 +180,7 @@ int replay(const Call& c, Report& r, std::vector<uint8_t>& written) {
             ++r.copies;
             for (int lane = 0; lane < 64; ++lane) {
               int key, col;
-              if (which) v_dma_source<D>(w * INSTS + ri, lane, &key, &col);
+              if (which) v_dma_source<D>(vl, w * INSTS + ri, lane, &key, &col);
               else k_dma_source<D>(w * INSTS + ri, lane, &key, &col);
               uint32_t voff;
               if (gather) {
@@ -187,8 +189,15 @@ int replay(const Call& c, Report& r, std::vector<uint8_t>& written) {
               } else {
                 voff = (uint32_t)(key * s_tok + col) * 2u;
               }
-              r.checks += 2;
+              r.checks += 3;
               const int lds = (w * INSTS + ri) * 1024 + lane * 16;
+              // where the kernel's operand reads look for this chunk
+              const int at = which && vl ? v_offset<D>(key, col) : s_offset<D>(key, col / 8);
+              if (key < 0 || key >= BN || col < 0 || col + 8 > D || at != lds) {
+                snprintf(msg, sizeof(msg), "item %d: %s key %d element %d copied to LDS byte %d, read at %d", item,
+                         which ? "V" : "K", key, col, lds, at);
+                r.fail(msg);
+              }
               if (lds < 0 || lds + 16 > TILE) {
                 snprintf(msg, sizeof(msg), "item %d: LDS write at %d of a %d-byte tile", item, lds, TILE);
                 r.fail(msg);
@@ -338,11 +347,11 @@ int64_t karpo_replay_pair_blocks(int waves, int insts, int64_t k_stride, int64_t
     for (int lane = 0; lane < 64; ++lane) {
       int k0, c0, v0, d0;
       k_dma_source<512>(w * insts, lane, &k0, &c0);
-      v_dma_source<512>(w * insts, lane, &v0, &d0);
+      v_dma_source<512>(true, w * insts, lane, &v0, &d0);
       for (int r = 0; r < insts; ++r) {
         int k, c, v, d;
         k_dma_source<512>(w * insts + r, lane, &k, &c);
-        v_dma_source<512>(w * insts + r, lane, &v, &d);
+        v_dma_source<512>(true, w * insts + r, lane, &v, &d);
         bad += (k * k_stride + c) * 2 != (k0 * k_stride + c0) * 2 + k_block * r;
         bad += (v * v_stride + d) * 2 != (v0 * v_stride + d0) * 2 + v_block * r;
       }

@@ -1,7 +1,7 @@
 """Host replay of the forward kernel's memory accesses (tests/replay/fwd_replay.cpp, built here with g++): for a call
 and its host plan, every workgroup, wave, lane and key step of the launch computes its addresses with the kernel's
-own functions (csrc/tile_addr.h, csrc/plan_common.h); each must stay inside its allocation, and every (query row,
-head) of every sequence must be written exactly once.
+own functions (csrc/tile_addr.h, csrc/plan_common.h); each must stay inside its allocation, every copied chunk must land
+where the operand reads look for it, and every (query row, head) of every sequence must be written exactly once.
 
 The row-table workloads are the ones behind the one GPU memory fault this build has seen (a block plan's branched
 pack read through its row table by the twelve-wave, 64-key tile at head size 128): their replay under that tile, and
@@ -135,6 +135,16 @@ def test_workloads_without_a_row_table(replay, name):
                                     w.window_right, spans=w.spans or (), max_q=w.max_q)
     assert bad == 0, first
     assert counts[4] == 0
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(32, 16, 128), (16, 8, 256), (8, 2, 64), (32, 4, 512)])
+def test_decode_shaped_tiles(replay, heads, kv_heads, head_dim):
+    """One query per sequence: the one-wave tiles that stream their keys (V in a layout of its own below head size 512),
+    every chunk copied to where the operand reads look for it."""
+    k_cu = [0, 1, 300, 333, 2000]
+    bad, counts, first = run_replay(replay, list(range(5)), k_cu, heads, kv_heads, head_dim, -1, -1, max_q=1)
+    assert bad == 0, first
+    assert counts[2] > 0 and counts[4] == 0
 
 
 def test_long_layer_with_split_tiles(replay):
