@@ -408,11 +408,12 @@ WideSizes wide_sizes_of(const KarpoAttnBwdArgs* b, const BwdSizes& z, size_t lim
   return w;
 }
 
-// The chunked path addresses a tile's 256 rows with 32-bit byte offsets.
+// The chunked path addresses a tile's 256 rows with 32-bit byte offsets, and reads all of its inputs by copies bounded by
+// rows * stride: nothing of rows that overlap (a gradient expanded over the rows), which the wave pairs' dQ reads whole.
 bool wide_strides(const KarpoAttnBwdArgs* b) {
   const int64_t strides[] = {b->fwd.q_stride_tok, b->fwd.k_stride_tok, b->fwd.v_stride_tok, b->d_o_stride_tok};
   for (int64_t s : strides)
-    if ((s + 512) * kWideTile * 2 >= (int64_t)INT32_MAX) return false;
+    if (s < 512 || (s + 512) * kWideTile * 2 >= (int64_t)INT32_MAX) return false;
   return true;
 }
 

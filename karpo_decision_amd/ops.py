@@ -525,7 +525,8 @@ def packed_attention_backward(grad: Tensor, query: Tensor, key: Tensor, value: T
     if lse.shape != (query.shape[1], query.shape[0]) or lse.dtype != torch.float32 or not lse.is_contiguous():
         raise ValueError("lse must be the forward's contiguous (heads, rows) fp32 tensor")
     lib = _lib.load()
-    grad = grad if grad.stride(-1) == 1 and grad.stride(0) % 8 == 0 and grad.stride(1) % 8 == 0 else grad.contiguous()
+    sg = grad.stride()  # (a gradient expanded over the rows is copied: the kernels' copies are bounded by rows * stride)
+    grad = grad if sg[2] == 1 and not (sg[0] | sg[1]) & 7 and sg[0] >= query.shape[2] else grad.contiguous()
     dq = torch.empty(query.shape, dtype=query.dtype, device=query.device)
     dk = torch.empty(key.shape, dtype=key.dtype, device=key.device)
     dv = torch.empty(value.shape, dtype=value.dtype, device=value.device)

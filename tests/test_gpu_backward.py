@@ -365,6 +365,24 @@ def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, k
             assert r < REL_FRO and rp < 2.0 ** -10, (form, name, r, rp)
 
 
+@pytest.mark.parametrize("heads,kv_heads,d", [(4, 2, 64), (4, 2, 128), (4, 2, 256), (8, 1, 512)])
+def test_gradient_expanded_over_the_rows(gpu, heads, kv_heads, d):
+    """An output gradient that is one row expanded over all rows (row stride 0), as the operator takes it: the same
+    gradients, bitwise, as from its contiguous copy."""
+    dev = torch.device("cuda")
+    n = 333
+    q, k, v, do, q_cu, _, _ = make_pack([n], [n], heads, kv_heads, d, seed=d)
+    q, k, v = (t.to(dev) for t in (q, k, v))
+    row = do[:1].to(dev)
+    cu = torch.tensor(q_cu, dtype=torch.int32, device=dev)
+    out, lse = ops.packed_attention_lse(q, k, v, cu, cu, n, d ** -0.5, -1, 0, None)
+    got = ops.packed_attention_backward(row.expand(n, heads, d), q, k, v, out, lse, cu, cu, n, d ** -0.5, -1, 0, None)
+    want = ops.packed_attention_backward(row.expand(n, heads, d).contiguous(), q, k, v, out, lse, cu, cu, n, d ** -0.5,
+                                         -1, 0, None)
+    for name, x, w in zip(("dq", "dk", "dv"), got, want):
+        assert float(w.float().abs().max()) > 0 and torch.equal(x, w), name
+
+
 def test_sliding_case_of_the_reference(gpu):
     """The reference's FA4 sliding test (tests/gpu/test_packed_gemma.py:70-104): head size 256, 32 / 16 heads, window
     1023, queries and keys with their own bounds (three branches after a shared tail), loss sum(out * linspace(-1, 1));

@@ -347,6 +347,14 @@ def test_bwd_workspace_holds_stats_and_both_plans():
     assert lib.karpo_attn_bwd(ctypes.byref(_bwd_args(_args(total_q=0, total_k=100))), None) == 0  # nothing to do
 
 
+def _bwd_512(heads, kv_heads, rows):
+    """One sequence of `rows` rows at head size 512, contiguous tensors."""
+    b = _bwd_args(_args(n_seq=1, heads=heads, kv_heads=kv_heads, head_dim=512, total_q=rows, max_q=rows, total_k=rows,
+                        q_stride_tok=heads * 512, k_stride_tok=kv_heads * 512, v_stride_tok=kv_heads * 512))
+    b.d_o_stride_tok = heads * 512
+    return b
+
+
 @pytest.mark.parametrize("heads,kv_heads,rows,chunked", [
     (32, 4, 16384, True), (32, 4, 131072, True),   # group 8: from 256 rows a chunk
     (32, 16, 65536, True),                         # group 2: chunks of 512 rows
@@ -358,11 +366,25 @@ def test_bwd_chunks_only_where_they_are_faster(heads, kv_heads, rows, chunked):
     """Head size 512, one sequence: the workspace of the chunked path (4 GiB of P and dS at most) only where its chunks
     are longer than those that lose to the wave pairs."""
     lib = _lib.load()
-    b = _bwd_args(_args(n_seq=1, heads=heads, kv_heads=kv_heads, head_dim=512, total_q=rows, max_q=rows, total_k=rows))
+    b = _bwd_512(heads, kv_heads, rows)
     least, best = ctypes.c_size_t(), ctypes.c_size_t()
     assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(least)) == 0
     assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(best)) == 0
     assert (best.value > least.value) == chunked, (least.value, best.value)
+
+
+@pytest.mark.parametrize("name", ["q", "k", "v", "d_o"])
+@pytest.mark.parametrize("stride,chunked", [(504, False), (0, False), (512, True), (4193784, True), (4193792, False)])
+def test_bwd_chunks_only_with_strides_they_address(name, stride, chunked):
+    """Head size 512, one sequence: rows that overlap (a gradient expanded over the rows) and tiles of 256 rows past 2^31
+    bytes keep the wave pairs."""
+    lib = _lib.load()
+    b = _bwd_512(8, 1, 600)
+    setattr(b if name == "d_o" else b.fwd, f"{name}_stride_tok", stride)
+    least, best = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(least)) == 0
+    assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(best)) == 0
+    assert (best.value > least.value) == chunked
 
 
 @pytest.mark.parametrize("room,free,steps", [
@@ -378,8 +400,7 @@ def test_bwd_workspace_when_memory_is_short(monkeypatch, room, free, steps):
     """16,384 rows of 32 / 4 heads at head size 512: the allocations that the backward tries (as divisors of the best
     size, 0: the least), with `room` bytes to be had and `free` reported; the largest that fits is returned."""
     lib = _lib.load()
-    rows = 16384
-    b = _bwd_args(_args(n_seq=1, heads=32, kv_heads=4, head_dim=512, total_q=rows, max_q=rows, total_k=rows))
+    b = _bwd_512(32, 4, 16384)
     least, best = ctypes.c_size_t(), ctypes.c_size_t()
     assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(least)) == 0
     assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(best)) == 0
