@@ -313,24 +313,86 @@ def test_head_512_one_sequence_cases_of_the_reference(gpu, causal):
             assert r < REL_FRO, ((lq, lk), name, r)
 
 
-@pytest.mark.parametrize("lq,lk,pad,heads,kv_heads,right", [
-    (1, 1, 3, 8, 4, 0),        # one row
-    (256, 256, 0, 8, 1, 0),    # exactly one tile
-    (513, 1000, 0, 16, 2, 0),  # one row past two tiles, keys not a multiple of a tile, Lk > Lq
-    (700, 333, 5, 8, 8, 0),    # Lq > Lk: rows and key tiles that see nothing
-    (400, 900, 0, 6, 3, -1),   # bidirectional, a head count that does not spread over the XCDs
-    (1030, 1030, 90, 8, 1, 70),  # keys ahead of the diagonal
-])
-def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, kv_heads, right):
-    """One sequence at head size 512: the path that keeps P and dS of a chunk of query rows in the workspace, in one
-    chunk and in chunks of 256 rows (the workspace that leaves room for no more), against the oracle's float32
-    gradients and the wave-pair kernels (which the least workspace selects). The workspace and the rows past the
-    sequence hold NaN, which reach no gradient. Both paths round P and dS to bf16 and sum in fp32, so each is within
-    REL_FRO of float32, and they differ only by the order of their fp32 sums: a rounding of P, dS or a result to bf16
-    may then fall the other way in a few elements, 2^-9 at most each, so below 2^-10 over the norm. (One key: dS is a
-    difference that cancels, only dV is compared.)"""
+# ---- one sequence at head size 512: the path that keeps P and dS of a chunk of query rows in the workspace
+
+def chunk_bytes(total_q, total_k, heads, kv_heads, rows):
+    """(statistics, P and dS of `rows` rows, dK and dV in fp32): the chunked path's workspace, in bytes."""
+    keys = -(-total_k // 256) * 256
+    return -(-heads * 2 * total_q * 4 // 256) * 256, 4 * rows * keys * heads, 2 * keys * kv_heads * 512 * 4
+
+
+def chunks_of(total_q, total_k, heads, kv_heads, size):
+    """Chunks that a workspace of `size` bytes leads to (all rows' P and dS in one where they fit)."""
+    rows = -(-total_q // 256) * 256
+    stats, scores, kept = chunk_bytes(total_q, total_k, heads, kv_heads, rows)
+    if stats + scores <= size:
+        return 1
+    most = (size - stats - kept) // (scores // rows) // 256 * 256
+    return -(-rows // most)
+
+
+def wide_forms(monkeypatch, call, total_q, total_k, heads, kv_heads, rows):
+    """`call()` with the least workspace (the wave pairs), with one that holds chunks of `rows` rows (None: not run) and
+    with the fastest path's. The workspace starts as NaN, and each form's use of it is checked: the least holds the wave
+    pairs' plan (32 keys a step, four waves) behind the statistics; the others P and dS there, and dK and dV in fp32 behind
+    those exactly if there is more than one chunk."""
     import ctypes
 
+    stats = chunk_bytes(total_q, total_k, heads, kv_heads, 256)[0]
+    got = {}
+    for form in ("least", "chunks", "best"):
+        if form == "chunks" and rows is None:
+            continue
+        kept = []
+
+        def workspace(lib, args, device):
+            least, best = ctypes.c_size_t(), ctypes.c_size_t()
+            assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(args), ctypes.byref(least)) == 0
+            assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(args), ctypes.byref(best)) == 0
+            assert best.value > least.value
+            chunked = sum(chunk_bytes(total_q, total_k, heads, kv_heads, rows)) if rows else 0
+            size = {"least": least.value, "chunks": max(least.value, chunked), "best": best.value}[form]
+            kept.append(torch.full((size,), 255, dtype=torch.uint8, device=device))
+            return kept[0]
+
+        monkeypatch.setattr(ops, "_backward_workspace", workspace)
+        print("head 512 one sequence", (total_q, total_k, heads, kv_heads), form, flush=True)
+        got[form] = call()
+        torch.cuda.synchronize()
+        ws = kept[0]
+        plan = ws[stats:stats + 48].view(torch.int32).tolist()
+        if form == "least":
+            assert plan[2] == 32 and plan[5] == 4, plan
+            continue
+        n = chunks_of(total_q, total_k, heads, kv_heads, ws.numel())
+        assert (n > 1) == (form == "chunks")
+        scores = chunk_bytes(total_q, total_k, heads, kv_heads, rows if n > 1 else -(-total_q // 256) * 256)[1]
+        assert bool((ws[stats:stats + scores] != 255).any())
+        assert bool((ws[stats + scores:] != 255).any()) == (n > 1)
+    return got
+
+
+@pytest.mark.parametrize("lq,lk,pad,heads,kv_heads,right,rows", [
+    (1, 1, 3, 8, 4, 0, None),          # one row
+    (256, 256, 0, 8, 1, 0, None),      # exactly one tile
+    (700, 333, 5, 8, 8, 0, None),      # Lq > Lk: rows and key tiles that see nothing
+    (400, 900, 0, 6, 3, -1, None),     # bidirectional, a head count that does not spread over the XCDs
+    (513, 1000, 0, 16, 2, 0, 256),     # one row past two chunks, keys not a multiple of a tile, Lk > Lq
+    (1030, 1030, 90, 8, 1, 70, 256),   # keys ahead of the diagonal
+    (1500, 333, 0, 8, 1, 0, 256),      # Lq > Lk over chunks: the first ones see nothing
+    (1500, 900, 0, 8, 1, -1, 256),     # bidirectional: every key tile carried into every later chunk
+    (600, 600, 300, 8, 1, 0, 256),     # chunks after the one that holds the last row
+    (1300, 1300, 0, 4, 2, 0, 512),     # group 2: chunks of 512 rows
+    (3000, 2950, 40, 4, 4, 0, 1024),   # group 1: of 1,024
+])
+def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, kv_heads, right, rows):
+    """One sequence at head size 512: the path that keeps P and dS of a chunk of query rows in the workspace, in one
+    chunk and in chunks of `rows` rows (three to six of them), against the oracle's float32 gradients and the wave-pair
+    kernels (which the least workspace selects). The workspace and the rows past the sequence hold NaN, which reach no
+    gradient. Both paths round P and dS to bf16 and sum in fp32, so each is within REL_FRO of float32, and they differ only
+    by the order of their fp32 sums: a rounding of P, dS or a result to bf16 may then fall the other way in a few
+    elements, 2^-9 at most each, so below 2^-10 over the norm. (One key: dS is a difference that cancels, only dV is
+    compared.)"""
     dev = torch.device("cuda")
     q, k, v, do, _, _, _ = make_pack([lq + pad], [lk + pad], heads, kv_heads, 512, seed=lq)
     want = oa.packed_grads(q[:lq], k[:lk], v[:lk], do[:lq], [0, lq], [0, lk], 0.05, -1, right, dtype=torch.float32)[1:]
@@ -339,30 +401,104 @@ def test_head_512_one_sequence_in_chunks(gpu, monkeypatch, lq, lk, pad, heads, k
     q, k, v, do = (t.to(dev) for t in (q, k, v, do))
     qc, kc = (torch.tensor([0, n], dtype=torch.int32, device=dev) for n in (lq, lk))
     out, lse = ops.packed_attention_lse(q, k, v, qc, kc, lq, 0.05, -1, right, None)
-    keys = -(-(lk + pad) // 256) * 256
-    # statistics, P and dS of 256 rows, dK and dV in fp32
-    chunk = -(-heads * 2 * (lq + pad) * 4 // 256) * 256 + 4 * 256 * keys * heads + 2 * keys * kv_heads * 512 * 4
-    got = {}
-    for form in ("least", "chunks", "best"):
-        def workspace(lib, args, device):
-            least, best = ctypes.c_size_t(), ctypes.c_size_t()
-            assert lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(args), ctypes.byref(least)) == 0
-            assert lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(args), ctypes.byref(best)) == 0
-            size = {"least": least.value, "chunks": max(least.value, chunk), "best": best.value}[form]
-            assert best.value >= size or form == "chunks"
-            return torch.full((size,), 255, dtype=torch.uint8, device=device)
-
-        monkeypatch.setattr(ops, "_backward_workspace", workspace)
-        print("head 512 one sequence", (lq, lk), form, flush=True)
-        got[form] = ops.packed_attention_backward(do, q, k, v, out, lse, qc, kc, lq, 0.05, -1, right, None)
-        torch.cuda.synchronize()
-        for name, x, w, pair in zip(("dq", "dk", "dv"), got[form], want, got["least"]):
+    got = wide_forms(monkeypatch, lambda: ops.packed_attention_backward(do, q, k, v, out, lse, qc, kc, lq, 0.05, -1, right,
+                                                                        None),
+                     lq + pad, lk + pad, heads, kv_heads, rows)
+    for form, grads in got.items():
+        for name, x, w, pair in zip(("dq", "dk", "dv"), grads, want, got["least"]):
             if lk == 1 and name != "dv":
                 continue
             n = w.shape[0]
             r, rp = rel(x[:n], w), rel(x[:n], pair[:n])
-            print("   ", name, f"rel {r:.2e}, against the pairs {rp:.2e}", flush=True)
+            print("   ", form, name, f"rel {r:.2e}, against the pairs {rp:.2e}", flush=True)
             assert r < REL_FRO and rp < 2.0 ** -10, (form, name, r, rp)
+
+
+@pytest.mark.parametrize("layout", ["head-major", "padded", "offset", "zero scale", "negative scale"])
+def test_head_512_one_sequence_layouts(gpu, monkeypatch, layout):
+    """The same path with heads outside rows, with padded rows and heads, with bounds that do not start at 0 (NaN on both
+    sides), and with a zero and a negative scale; 900 rows over 700 keys, in chunks of 256 and in one. Compared as above;
+    at scale 0 dQ and dK are exact zeros (a product with the scale)."""
+    dev = torch.device("cuda")
+    lq, lk, heads, kv_heads = 900, 700, 8, 1
+    scale = {"zero scale": 0.0, "negative scale": -0.05}.get(layout, 0.05)
+    q0, k0 = (37, 11) if layout == "offset" else (0, 0)
+    q, k, v, do, _, _, _ = make_pack([lq], [lk], heads, kv_heads, 512, seed=5)
+    want = oa.packed_grads(q, k, v, do, [0, lq], [0, lk], scale, -1, 0, dtype=torch.float32)[1:]
+
+    def place(t, first):
+        n, h, d = t.shape
+        if layout == "head-major":
+            return t.to(dev).permute(1, 0, 2).contiguous().permute(1, 0, 2)
+        if layout == "padded":
+            x = torch.full((n, h + 1, d + 8), float("nan"), dtype=t.dtype, device=dev)[:, :h, :d]
+        else:
+            x = torch.full((n + 2 * first, h, d), float("nan"), dtype=t.dtype, device=dev)
+        x[first:first + n] = t.to(dev)
+        return x
+
+    q, do, k, v = place(q, q0), place(do, q0), place(k, k0), place(v, k0)
+    qc = torch.tensor([q0, q0 + lq], dtype=torch.int32, device=dev)
+    kc = torch.tensor([k0, k0 + lk], dtype=torch.int32, device=dev)
+    out, lse = ops.packed_attention_lse(q, k, v, qc, kc, lq, scale, -1, 0, None)
+    got = wide_forms(monkeypatch, lambda: ops.packed_attention_backward(do, q, k, v, out, lse, qc, kc, lq, scale, -1, 0,
+                                                                        None),
+                     q.shape[0], k.shape[0], heads, kv_heads, 256)
+    for form, grads in got.items():
+        for name, x, w, pair, first in zip(("dq", "dk", "dv"), grads, want, got["least"], (q0, k0, k0)):
+            x, pair = x[first:first + w.shape[0]], pair[first:first + w.shape[0]]
+            if scale == 0 and name != "dv":
+                assert not x.any(), (form, name)
+                continue
+            r, rp = rel(x, w), rel(x, pair)
+            print("   ", layout, form, name, f"rel {r:.2e}, against the pairs {rp:.2e}", flush=True)
+            assert r < REL_FRO and rp < 2.0 ** -10, (form, name, r, rp)
+
+
+def test_head_512_one_sequence_short_chunks_keep_the_wave_pairs(gpu, monkeypatch):
+    """A workspace with room for chunks of 512 rows only, at a group of 1: the wave pairs run (their plan behind the
+    statistics), bitwise as with the least workspace."""
+    dev = torch.device("cuda")
+    n, heads = 3000, 4
+    q, k, v, do, q_cu, _, _ = make_pack([n], [n], heads, heads, 512, seed=3)
+    q, k, v, do = (t.to(dev) for t in (q, k, v, do))
+    cu = torch.tensor(q_cu, dtype=torch.int32, device=dev)
+    out, lse = ops.packed_attention_lse(q, k, v, cu, cu, n, 0.05, -1, 0, None)
+    sizes = chunk_bytes(n, n, heads, heads, 512)
+    got = []
+    for more in (0, sum(sizes)):
+        kept = []
+
+        def workspace(lib, args, device):
+            kept.append(ops._workspace(lib, lib.karpo_attn_bwd_workspace_bytes, args, device))
+            assert kept[0].numel() < sum(sizes)
+            if more:
+                kept[0] = torch.full((more,), 255, dtype=torch.uint8, device=device)
+            return kept[0]
+
+        monkeypatch.setattr(ops, "_backward_workspace", workspace)
+        got.append(ops.packed_attention_backward(do, q, k, v, out, lse, cu, cu, n, 0.05, -1, 0, None))
+        plan = kept[0][sizes[0]:sizes[0] + 48].view(torch.int32).tolist()
+        assert plan[2] == 32 and plan[5] == 4, plan
+    for x, y in zip(*got):
+        assert torch.equal(x, y)
+
+
+def test_head_512_one_sequence_past_the_strides(gpu):
+    """Rows 4 Mi elements apart (a tile of 256 of them passes 2^31 bytes): refused by the chunked path, run by the wave
+    pairs, the gradients those of the contiguous tensors through them."""
+    dev = torch.device("cuda")
+    n, heads = 5, 8
+    q, k, v, do, q_cu, _, _ = make_pack([n], [n], heads, 1, 512, seed=9)
+    want = oa.packed_grads(q, k, v, do, q_cu, q_cu, 0.05, -1, 0, dtype=torch.float32)[1:]
+    far = torch.zeros((n, 1 << 22), dtype=torch.bfloat16, device=dev)[:, :heads * 512].view(n, heads, 512)
+    far.copy_(q)
+    k, v, do = (t.to(dev) for t in (k, v, do))
+    cu = torch.tensor(q_cu, dtype=torch.int32, device=dev)
+    out, lse = ops.packed_attention_lse(far, k, v, cu, cu, n, 0.05, -1, 0, None)
+    got = ops.packed_attention_backward(do, far, k, v, out, lse, cu, cu, n, 0.05, -1, 0, None)
+    for name, x, w in zip(("dq", "dk", "dv"), got, want):
+        assert rel(x, w) < REL_FRO, name
 
 
 @pytest.mark.parametrize("heads,kv_heads,d", [(4, 2, 64), (4, 2, 128), (4, 2, 256), (8, 1, 512)])

@@ -1,10 +1,11 @@
 """The backward (karpo_attn_bwd) at the sizes it is measured at, against the CPU oracle on an MI355X.
 
-Four layers, each run whole through the C ABI (the forward's output and log-sum-exp from ``packed_attention_lse``,
+Four layers (one of them twice), each run whole through the C ABI (the forward's output and log-sum-exp from ``packed_attention_lse``,
 then ``karpo_attn_bwd`` into NaN-filled dQ, dK and dV): the 32k-token global layer (32 / 16 heads, head_dim 128,
 causal; its dK / dV in the two-group kernel), the 16k sliding layer (16 / 8 heads, head_dim 256, window 1023), the Qwen
-8k pack (16 / 8 heads, head_dim 128, causal) and the 31B global layer (32 / 4 heads, head_dim 512, causal, the pair
-kernels). Checks:
+8k pack (16 / 8 heads, head_dim 128, causal) and the 31B global layer (32 / 4 heads, head_dim 512, causal): with the
+least workspace in the pair kernels, and with the fastest path's as the operator runs it, P and dS of 32 chunks of 1,024
+query rows in 4 GiB (byte offsets past 2^31). Checks:
 
 * every (row, head) of dQ, dK and dV is written and finite;
 * the first and the last key/value head group (the key/value head and its query heads: their gradients depend on no
@@ -27,7 +28,7 @@ from oracle import attention as oa
 pytestmark = pytest.mark.gpu
 
 REL_FRO = 1e-2
-LAYERS = ("global32k", "sliding", "qwen", "global32k_d512")
+LAYERS = ("global32k", "sliding", "qwen", "global32k_d512", "global32k_d512/chunks")
 
 
 def rel(a: torch.Tensor, b: torch.Tensor) -> float:
@@ -35,8 +36,9 @@ def rel(a: torch.Tensor, b: torch.Tensor) -> float:
     return float((a - b).norm() / b.norm().clamp_min(1e-30))
 
 
-def _backward_c_abi(w, do, out, lse, q_cu, k_cu, spans):
-    """karpo_attn_bwd into NaN-filled gradient buffers (a row it skipped stays NaN)."""
+def _backward_c_abi(w, do, out, lse, q_cu, k_cu, spans, best):
+    """karpo_attn_bwd into NaN-filled gradient buffers (a row it skipped stays NaN), with the least workspace or (``best``)
+    the fastest path's."""
     lib = _lib.load()
     q, k, v = w.query, w.key, w.value
     dq, dk, dv = (torch.full_like(t, float("nan")) for t in (q, k, v))
@@ -51,6 +53,10 @@ def _backward_c_abi(w, do, out, lse, q_cu, k_cu, spans):
     b.d_v, b.d_v_stride_tok, b.d_v_stride_head = dv.data_ptr(), dv.stride(0), dv.stride(1)
     need = ctypes.c_size_t()
     _lib.check(lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(need)), "workspace")
+    least = need.value
+    if best:
+        _lib.check(lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(need)), "workspace")
+        assert need.value > 4 << 30 > least
     ws = torch.full((need.value,), 0x7F, dtype=torch.uint8, device=q.device)  # garbage: nothing may rely on zeros
     b.fwd.workspace, b.fwd.workspace_bytes = ws.data_ptr(), need.value
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -62,7 +68,8 @@ def _backward_c_abi(w, do, out, lse, q_cu, k_cu, spans):
 @functools.lru_cache(maxsize=None)  # host copies of the compared heads only: the layer's GPU tensors are freed
 def _layer(name: str):
     dev = torch.device("cuda", 0)
-    w = workloads.named(name, dev, seed=0)
+    base, _, form = name.partition("/")
+    w = workloads.named(base, dev, seed=0)
     gen = torch.Generator(device=dev)
     gen.manual_seed(99)
     do = torch.randn(w.query.shape, generator=gen, device=dev).bfloat16()
@@ -74,7 +81,7 @@ def _layer(name: str):
         out, lse = ops.packed_attention_lse(w.query, w.key, w.value, q_cu, k_cu, w.max_q, w.scale, w.window_left,
                                             w.window_right, spans)
     print(f"layer {name}: backward through the C ABI", flush=True)
-    dq, dk, dv = _backward_c_abi(w, do, out, lse, q_cu, k_cu, spans)
+    dq, dk, dv = _backward_c_abi(w, do, out, lse, q_cu, k_cu, spans, form == "chunks")
     written = {n: bool(torch.isfinite(t).all()) for n, t in (("dq", dq), ("dk", dk), ("dv", dv))}
     group = w.heads // w.kv_heads
     keep = {}
@@ -94,11 +101,11 @@ def test_every_gradient_row_is_written(gpu, name):
 
 
 @functools.lru_cache(maxsize=None)
-def _oracle(name: str, g: int, dtype: torch.dtype):
-    layer = _layer(name)
+def _oracle(base: str, g: int, dtype: torch.dtype):
+    layer = _layer(base)
     q_cu, k_cu, scale, left, right, spans, _ = layer["w"]
     q, k, v, do = layer["groups"][g]["inputs"]
-    print(f"layer {name}: oracle ({dtype}) for key/value head {g}", flush=True)
+    print(f"layer {base}: oracle ({dtype}) for key/value head {g}", flush=True)
     return oa.packed_grads(q, k, v, do, q_cu, k_cu, scale, left, right, spans, dtype=dtype)
 
 
@@ -113,7 +120,7 @@ def test_head_group_gradients_match_the_oracle(gpu, name, which):
     relative Frobenius error below 1e-2."""
     g = _group(name, which)
     got = _layer(name)["groups"][g]["got"]
-    want = _oracle(name, g, torch.float32)
+    want = _oracle(name.partition("/")[0], g, torch.float32)
     for label, x, w in zip(("out", "dq", "dk", "dv"), got, want):
         r = rel(x, w)
         print(name, g, label, f"rel {r:.2e}", flush=True)
@@ -127,8 +134,8 @@ def test_head_group_gradients_within_twice_the_bf16_error(gpu, name, which):
     oracle): the reference's criterion for its backward kernels."""
     g = _group(name, which)
     got = _layer(name)["groups"][g]["got"]
-    want = _oracle(name, g, torch.float32)
-    base = _oracle(name, g, torch.bfloat16)
+    want = _oracle(name.partition("/")[0], g, torch.float32)
+    base = _oracle(name.partition("/")[0], g, torch.bfloat16)
     for label, x, w, b in zip(("out", "dq", "dk", "dv"), got, want, base):
         r, rb = rel(x, w), rel(b, w)
         print(name, g, label, f"rel {r:.2e} (oracle bf16 {rb:.2e})", flush=True)
