@@ -48,8 +48,7 @@ def parse() -> argparse.Namespace:
                         "them (the reference's Packed._gather path) instead of reading through the table")
     p.add_argument("--backward", action="store_true",
                    help="time the backward (karpo_attn_bwd: dq, dk, dv from the output gradient, the forward's "
-                        "output and log-sum-exp) instead of the forward; head sizes 64, 128 and 256, no gather or "
-                        "fused prologue")
+                        "output and log-sum-exp) instead of the forward; no gather or fused prologue")
     p.add_argument("--copy-bytes", type=int, default=0,
                    help="after the timed steps, copy this many bytes device to device once (a calibration kernel of "
                         "known traffic for rocprofv3 FETCH_SIZE / WRITE_SIZE)")
@@ -195,10 +194,43 @@ def cpu_backward_baseline(w) -> dict:
                        f"{sec:.3f} s; os.cpu_count()={os.cpu_count()}")}
 
 
+def backward_kernels(w, step) -> list[str]:
+    """The kernels that one backward step launches. At head size 512 the workspace that the operator got tells the path
+    (the fastest's where the library has one for the call and the device had the memory)."""
+    import ctypes
+
+    from karpo_decision_amd import ops
+
+    if w.head_dim != 512:
+        return [f"bwd_dq_kernel<{w.head_dim}>",
+                "bwd_dkdv2_kernel<128>" if w.head_dim == 128 else f"bwd_dkdv_kernel<{w.head_dim}>"]
+    sizes, real = [], ops._backward_workspace
+
+    def workspace(lib, b, device):
+        got, least, best = real(lib, b, device), ctypes.c_size_t(), ctypes.c_size_t()
+        lib.karpo_attn_bwd_workspace_bytes(ctypes.byref(b), ctypes.byref(least))
+        lib.karpo_attn_bwd_workspace_best_bytes(ctypes.byref(b), ctypes.byref(best))
+        sizes.append((least.value, got.numel(), best.value))
+        return got
+
+    ops._backward_workspace = workspace
+    try:
+        step()
+    finally:
+        ops._backward_workspace = real
+    least, got, best = sizes[0]
+    chunks, pairs = ["bwd_wide_ds_kernel", "bwd_wide_grad_kernel"], ["bwd_dq_pair_kernel<512>", "bwd_dkdv_pair_kernel<512>"]
+    if got == least:
+        return ["bwd_stats_kernel<512>", *pairs]
+    if got == best:
+        return ["bwd_stats_kernel<512>", *chunks]
+    return ["bwd_stats_kernel<512>", "by chunks or wave pairs: less workspace than the fastest path's"]
+
+
 def backward(args, device, w) -> int:
     """One step = karpo_attn_bwd over the pack (the planner launch for both work lists, the dq kernel, which also
-    writes the per-row statistics, and the dk/dv kernels; at head size 512 a statistics pass first and the wave-pair
-    kernels) from a resident output gradient, output and log-sum-exp. TFLOP/s counts the algorithmic
+    writes the per-row statistics, and the dk/dv kernels; at head size 512 a statistics pass first, then for one sequence
+    without a left window bound or spans the products of chunks of rows, the wave-pair kernels otherwise) from a resident output gradient, output and log-sum-exp. TFLOP/s counts the algorithmic
     backward: 2.5x the forward's FLOPs (five products per visible pair: S, dP, dV, dQ, dK)."""
     import torch
 
@@ -218,6 +250,7 @@ def backward(args, device, w) -> int:
         return ops.packed_attention_backward(grad, w.query, w.key, w.value, out, lse, q_cu, k_cu, w.max_q, w.scale,
                                              w.window_left, w.window_right, spans)
 
+    kernels = backward_kernels(w, step)
     for _ in range(args.warmup):
         step()
     torch.cuda.synchronize()
@@ -247,10 +280,7 @@ def backward(args, device, w) -> int:
                    "flops_per_step": flops, "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4), "traffic": None,
-                     "kernel": (f"karpo_attn_bwd (bwd_stats_kernel<512>, bwd_wide_ds_kernel, bwd_wide_grad_kernel)"
-                                if w.head_dim == 512 else
-                                f"karpo_attn_bwd (bwd_dq_kernel<{w.head_dim}>, "
-                                f"bwd_dkdv_kernel<{w.head_dim}, *>)"),
+                     "kernel": f"karpo_attn_bwd ({', '.join(kernels)})",
                      "avg_launch_ms": round(launch_ms, 4)},
     }
     if not args.no_cpu_baseline:
