@@ -169,7 +169,9 @@ int karpo_attn_norm_rope(const KarpoNormRopeArgs* args, void* stream);
  * 256 and 512; no plan, no row table, no prologue or gate in fwd (their gradients are other ops'). Gradient tensors
  * are bf16 with head_dim contiguous; every row inside the sequences' bounds (q_cu, k_cu) is written, rows outside
  * them are not. Deterministic: a key/value head's gradients sum over its query heads, and the parts of a key tile the
- * device planner splits over its query rows (head sizes 64, 128) in part order, each in a fixed order (no atomics). */
+ * device planner splits over its query rows (head sizes 64, 128) in part order, each in a fixed order (no atomics).
+ * Non-finite inputs are not confined to the pairs that see them: a pair outside the mask has a weight of exactly zero,
+ * and tiles compute with it (up to 256 query rows by 32 keys for d_q, 256 keys by 32 query rows for d_k and d_v). */
 typedef struct KarpoAttnBwdArgs {
   KarpoAttnArgs fwd;            /* the forward call's arguments (o = its output); fwd.total_k = rows of k and v;
                                    fwd.workspace / workspace_bytes: karpo_attn_bwd_workspace_bytes of these args */

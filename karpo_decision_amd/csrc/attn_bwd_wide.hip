@@ -7,10 +7,11 @@
 // of waves that exchange partial sums through LDS, one wave per SIMD, three barriers per 32-row step, 24-26% of the
 // MFMA rate), and it computes S and dP twice (seven products). P and dS cost 10 bytes of traffic per visible pair and
 // 5,120 FLOPs need them, so keeping them takes less time than either the recomputation or the exchange: five products,
-// each a plain tiled matrix product with every accumulator in one wave's registers. Measured against the wave pairs
-// (32 / 4 heads, causal, MI355X): 427 -> 121 us at 512 rows, 1.79 -> 0.64 ms at 2,048, 10.6 -> 6.1 ms at 8,192, 48.1 ->
-// 23.2 ms at 16,384; faster at every size tried (64 to 16,384 rows, 8 / 1, 32 / 4 and 32 / 16 heads), so every such
-// call takes this path when the workspace has room for a chunk of 256 rows.
+// each a plain tiled matrix product with every accumulator in one wave's registers. Measured against the wave pairs as
+// they are now (32 / 4 heads, causal, MI355X): 838 -> 253 us at 1,024 rows, 1.80 -> 0.63 ms at 2,048, 10.7 -> 6.1 ms at
+// 8,192, 41 -> 23 ms at 16,384. In one chunk it is faster at every size tried (1 to 16,384 rows over 1 to 65,536 keys,
+// groups 1 to 16), in several where they are long enough (wide_chunks_pay, capi.cpp); such calls take this path when the
+// workspace has room for it.
 //
 // P and dS in the workspace: per head [key block of 16][chunk of 8 rows][16 keys][8 rows] bf16, the 16 keys of a
 // 256-byte run XOR-swizzled by the chunk index (key ^ 4 (chunk % 4): free of bank conflicts read either way), the layout
@@ -20,7 +21,13 @@
 //
 // Chunks of rows run in ascending order. dQ of a chunk's rows is complete within it; dK and dV go on from one chunk to
 // the next in fp32 (workspace, in the accumulators' register order) and are rounded once, in the last chunk.
-// Every sum has a fixed order (no atomics): repeated calls are bitwise equal.
+// Every sum has a fixed order (no atomics): repeated calls with the same chunk size are bitwise equal (it sets where dK's
+// and dV's sums pass from one head of a group to the next).
+//
+// Outside the mask P and dS are exact zeros, and those enter the products with whatever the other operand holds: a NaN or
+// infinity in a K row reaches dQ of every row of the 256-row tiles that visit its 32-key step, one in a Q or dO row
+// dK or dV of the 256-key tiles that visit its 32-row step (the wave pairs: tiles of 64 query vectors, and of 64
+// keys). One in a V row reaches only dQ of the rows that see it. Rows past the sequence are never read.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -41,7 +48,7 @@ constexpr int kGradThreads = 256;               // kernel 2: four waves
 constexpr int kDsRows = 256, kDsKeys = 128;     // kernel 1's tile
 constexpr int kDsStep = 32;                     // elements of D per step
 constexpr int kGradTile = 256, kGradStep = 32;  // kernel 2's outputs (both ways) and contraction step
-constexpr int kRing = 4;                        // buffers: three steps of copies in flight
+constexpr int kRing = 4;                        // buffers: three steps of copies ahead
 
 // The sequence's bounds, clamped to the call's rows.
 struct WideSeq {
@@ -76,7 +83,11 @@ __device__ __forceinline__ void step_barrier() { asm volatile("s_waitcnt lgkmcnt
 
 // ---- kernel 1: P and dS of 256 rows x 128 keys of one head (eight waves of 64 x 64), for a run of key tiles: the next
 // tile's first copies are in flight while this one's P and dS are formed and stored, and a tile's exponentials run
-// beside its dP products
+// beside its dP products. 770 TFLOP/s over the eight chunks of 16,384 rows (32 / 4 heads), 40% MFMA-busy: bound by its
+// copies and stores, which overlap the products badly (the last chunk: 2.5 ms; without its copies 1.67, its copies alone
+// 1.71). Besides the waits below the compiler adds its own before the LDS reads of a tile's first three steps after
+// another tile (vmcnt 19, 12, 11: it does not follow which copy fills which buffer), so most of the 16 stores are waited for
+// there; and 176 SGPRs are spilled to VGPR lanes (171 lane moves in the tile loop).
 __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_ds_kernel(BwdWideParams w) {
   constexpr int STEPS = kWideD / kDsStep;  // per product
   constexpr int ALL = 2 * STEPS;           // S, then dP
@@ -276,7 +287,9 @@ __global__ __launch_bounds__(kWideThreads, 2) void bwd_wide_ds_kernel(BwdWidePar
 // four waves of 128 x 128 (one per SIMD, 256 accumulators in AGPRs): each operand read from LDS feeds four MFMAs. The
 // operands of a half step (16 of the contraction) are read during the MFMAs of the half step before it; the barrier
 // that publishes a step's copies is passed halfway through the step before, when every wave has read the whole of
-// that step's buffer, so the copies of three to four steps are in flight. The chunk of the last 2,048 of 16,384 rows
+// that step's buffer, so the copies of three to four steps are in flight. (dQ's loop drains them once in four steps: the
+// compiler puts a vmcnt(0) of its own before the first LDS read of the unrolled four; the dK / dV loop has none.) The
+// 65 spilled VGPRs are outside the loops. The chunk of the last 2,048 of 16,384 rows
 // (32 / 4 heads): 3.13 ms with eight waves of 128 x 64, 2.88 ms so, 2.50 ms with the reads and copies spread between the
 // MFMAs (sched_group_barrier); 1.4 ms at the nominal MFMA rate.
 template <bool DQ>
@@ -508,8 +521,11 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_wide_grad_kernel(BwdWideP
   const WideSeq s(w);
   // dK and dV first where the group is large: their items are then the longer ones (rows / 32 steps of every head of the
   // group, against the visible keys / 32 of dQ), and early chunks have few of them, so dQ fills the CUs that they leave
-  // free. Backward at 32 / 4 heads: 697 -> 637 us at 2,048 rows, 1.91 -> 1.80 ms at 4,096, 6.21 -> 6.11 at 8,192; at
-  // 32 / 16 heads (group 2) 1-2% slower at 4,096 and 8,192 rows.
+  // free. Backward in us, dQ first and dK / dV first (medians of seven in turn), at 1,024, 2,048, 4,096, 8,192 rows:
+  //   group 16 (32 / 2 heads): 394 379, 981 916, 2493 2318, 6948 6697     8 (32 / 4): 270 255, 706 639, 1942 1734, 6323 6013
+  //   4 (32 / 8): 209 196, 576 517, 1711 1699, 6032 6025                   4 (4 / 1): 112 112, 217 216, 447 447, 1334 1319
+  //   3 (24 / 8): 146 145, 426 390, 1368 1364, 4762 4725                   3 (6 / 2): 101 100, 204 205, 473 483, 1573 1507
+  //   2 (32 / 16): 184 180, 542 538, 1764 1768, 6452 6482                  1 (32 / 32): 203 205, 635 629, 2045 2073, 7443 7485
   const int dkdv_items = w.keys / kGradTile * 4 * (w.b.heads / w.b.group);
   const int dq_items = w.rows / kGradTile * 2 * w.b.heads;
   const bool dkdv_first = w.b.group >= 4;
@@ -521,7 +537,10 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_wide_grad_kernel(BwdWideP
 
 hipError_t launch_bwd_wide(BwdWideParams w, hipStream_t stream) {
   const int kv_heads = w.b.heads / w.b.group;
-  // key tiles per workgroup of kernel 1: at least 1,024 workgroups (four per CU), at most eight tiles
+  // key tiles per workgroup of kernel 1: at least 1,024 workgroups (four per CU), at most eight tiles. The backward of
+  // 16,384 rows at 32 / 4 heads with at most 1, 2, 4, 8, 16: 24.1, 22.9, 22.6, 22.8, 23.4 ms; 32 / 16: 27.1, 26.1, 25.8, 26.0,
+  // 26.7. At least 256, 512, 1,024, 2,048 workgroups: 264, 264, 251, 252 us at 1,024 rows (32 / 4), 995, 995, 932, 903 at 4,096
+  // (8 / 1), no difference where there are plenty.
   const int64_t row_tiles = (int64_t)(w.rows / kDsRows) * w.b.heads, key_tiles = w.keys / kDsKeys;
   const int64_t per = row_tiles * key_tiles / 1024;
   w.run = (int32_t)(per < 1 ? 1 : per > 8 ? 8 : per);

@@ -257,11 +257,12 @@ __global__ __launch_bounds__((64 * TileCfg<D, SHAPE>::W), (TileCfg<D, SHAPE>::OC
   static_assert(BLKS >= 1, "a tile holds at least one DMA instruction");
   static_assert(!PAIR || QB == 1, "a pair holds one query block");
 
-  // K/V buffers: NB - 1 steps of copies in flight. One-wave tiles that stream their keys (decode-shaped packs, HBM
-  // bound) keep three steps in flight in 64 KiB (two workgroups per CU: 96 KiB of copies in flight per CU instead of
-  // five workgroups' 80; the markers layer's attention kernel 115.9 -> 109.6 us, planned two per CU either way); the
-  // others two buffers. The deeper ring counts its own copies to wait for one step's, so it is only built where every
-  // copy instruction is issued unconditionally (one wave, no row table).
+  // K/V buffers: copies are issued NB - 1 steps ahead. One-wave tiles that stream their keys (decode-shaped packs, HBM
+  // bound) have four in 64 KiB, two workgroups per CU (the markers layer's attention kernel 115.9 -> 109.6 us against
+  // five double-buffered ones, planned two per CU either way); the others two buffers. The deeper ring counts its own copies
+  // to wait for one step's, so it is only built where every copy instruction is issued unconditionally (one wave, no row
+  // table). As compiled its counted wait is followed by the fence of __syncthreads, in a one-wave workgroup a vmcnt(0)
+  // without a barrier: a step ends when all issued copies have landed, and only the newest step's are in flight.
   constexpr int NB = kv_buffers(D, SHAPE, GATHER);
   static_assert(NB == 2 || (W == 1 && BLKS == INSTS), "the ring waits on a fixed count of its wave's copies");
   constexpr int CPS = 2 * INSTS;  // copy instructions per step of a one-wave tile (K and V)

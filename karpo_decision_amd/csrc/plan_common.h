@@ -124,9 +124,9 @@ KA_HD inline Geometry geometry(int heads, int kv_heads, int head_dim, int64_t ma
   return geometry_of(heads, kv_heads, head_dim, tile_shape(heads, kv_heads, head_dim, max_q, gather));
 }
 
-// K/V buffers of the forward kernel's ring (steps of copies in flight: buffers - 1). One-wave tiles that stream
-// their keys without a row table (decode-shaped packs, HBM bound) keep three steps in flight at head_dim 64 and 128
-// (four buffers); every other tile double-buffers.
+// K/V buffers of the forward kernel's ring (copies are issued buffers - 1 steps ahead). One-wave tiles that stream
+// their keys without a row table (decode-shaped packs, HBM bound) have four at head_dim 64 and 128; every other tile
+// double-buffers.
 KA_HD constexpr int kv_buffers(int head_dim, int shape, bool gather) {
   return shape == kNarrow && tile_waves(head_dim, shape) == 1 && !gather && head_dim <= 128 ? 4 : 2;
 }
