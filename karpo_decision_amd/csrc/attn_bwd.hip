@@ -631,7 +631,7 @@ __global__ __launch_bounds__(64 * kBwdWaves, 1) void bwd_dkdv_kernel(BwdParams p
 // the tile's rows (group 0 steps 0, 2, .., group 1 steps 1, 3, ..). K and V of the tile sit in LDS (the S layout,
 // read as the B operands of S = Q K^T and dP = dO V^T) instead of registers, which leaves room for both fp32
 // accumulators at 256 registers; at the end group 1's sums are added to group 0's through LDS in a fixed order
-// (repeated calls stay bitwise equal). Four products per step instead of the five of the dV and dK launches.
+// (repeated calls stay bitwise equal). Four products per step.
 template <int D>
 __global__ __launch_bounds__(64 * 2 * kBwdWaves, 2) void bwd_dkdv2_kernel(BwdParams p) {
   constexpr int KW = kBwdWaves, W = 2 * KW, BQ = kBwdStep;

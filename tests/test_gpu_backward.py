@@ -211,7 +211,7 @@ def test_long_key_tiles_split_over_their_query_steps(gpu, monkeypatch, q_lens):
     merges = ws[plan_k + 12: plan_k + 12 + 4 * header[4]].view(-1, 4).tolist()
     assert all(seg == 0 and parts >= 2 for seg, _, parts, _ in merges)  # the long sequence's tiles
     tiles_k = -(-sum(q_lens) // 128) + n_seq
-    assert (tiles_k * kv_heads >= 2048) == (len(q_lens) > 10)  # the two-launch path's threshold
+    assert (tiles_k * kv_heads >= 2048) == (len(q_lens) > 10)  # one pack of few key tiles, one of many
     want = oa.packed_grads(q, k, v, do, q_cu, k_cu, d ** -0.5, -1, 0, spans, dtype=torch.float32)
     for name, x, w in zip(("out", "dq", "dk", "dv"), got, want):
         r = rel(x, w)
