@@ -445,11 +445,15 @@ def _workspace(lib, fn, args, device: torch.device) -> Tensor:
 
 
 def _free_bytes(device: torch.device) -> int | None:
-    """Bytes the device could still give this process (free, or free in torch's cache); None during a graph capture."""
+    """Bytes the device could still give this process (free, or free in torch's cache); None where that is not known
+    (during a graph capture, or with an allocator that keeps no statistics)."""
     if torch.cuda.is_current_stream_capturing():
         return None
-    stats = torch.cuda.memory_stats_as_nested_dict(device)
-    cached = stats["reserved_bytes"]["all"]["current"] - stats["allocated_bytes"]["all"]["current"]
+    try:
+        stats = torch.cuda.memory_stats_as_nested_dict(device)
+        cached = stats["reserved_bytes"]["all"]["current"] - stats["allocated_bytes"]["all"]["current"]
+    except (KeyError, RuntimeError):
+        return None
     return torch.cuda.mem_get_info(device)[0] + cached
 
 

@@ -419,6 +419,28 @@ def test_bwd_workspace_when_memory_is_short(monkeypatch, room, free, steps):
     assert asked == [best.value // s if s else least.value for s in steps]
 
 
+def test_free_bytes_are_unknown_without_statistics(monkeypatch):
+    """During a capture, and with an allocator that has no statistics (torch's pluggable ones raise), the free memory is
+    not known: the workspace is then simply tried."""
+    def none(device):
+        raise RuntimeError("the allocator does not support getDeviceStats")
+
+    def stats(device):
+        return {"reserved_bytes": {"all": {"current": 900}}, "allocated_bytes": {"all": {"current": 500}}}
+
+    device = torch.device("cuda", 0)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device: (7000, 9000))
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", stats)
+    assert ops._free_bytes(device) == 7400
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", none)
+    assert ops._free_bytes(device) is None
+    monkeypatch.setattr(torch.cuda, "memory_stats_as_nested_dict", lambda device: {})
+    assert ops._free_bytes(device) is None
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert ops._free_bytes(device) is None
+
+
 def test_empty_pack_is_a_no_op():
     lib = _lib.load()
     assert lib.karpo_attn_fwd(ctypes.byref(_args(total_q=0)), None) == 0
